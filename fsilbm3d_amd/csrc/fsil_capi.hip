@@ -314,8 +314,9 @@ Block *get_block(int h) {
 // the warm-start network (fsil_mlp_kernels.h), one per handle
 struct Mlp {
   DevBuf<float> th, g, m, v;                         // parameters, gradient, Adam moments
-  DevBuf<float> X, Y, bx, by, H1, H2, H3, Yp, dY, dZ3, dZ2, dZ1;
-  DevBuf<double> part;
+  DevBuf<float> X, Y, Yp, gpart;                     // rows, outputs, the workgroups' gradient parts
+  DevBuf<double> part;                               // the workgroups' squared errors
+  int nblk = 0;                                      // workgroups of the last gradient pass
   DevBuf<int> idx;
   int adam_t = 0;
   hipStream_t s = nullptr;
@@ -1652,7 +1653,7 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
   if (warm) {
     // the learned guess of the force after `skip` rounds, applied to the band
     // as one correction of the uncorrected velocity
-    hipLaunchKernelGGL(k_mlp_infer_bf16, dim3((M + 63) / 64), dim3(256), 0, s, I.wsX.p, M, net->th.p, I.wsP.p);
+    hipLaunchKernelGGL(k_mlp_infer_bf16, dim3(std::min(kInferBlocks, (M + 63) / 64)), dim3(256), 0, s, I.wsX.p, M, net->th.p, I.wsP.p);
     hipLaunchKernelGGL(k_ws_apply, dim3((3 * M + 255) / 256), dim3(256), 0, s, M, I.wsP.p, I.Ea.p, I.Eprev.p, I.Uref,
                        invh3p, I.Eforce.p, I.fT.p);
     hipLaunchKernelGGL(k_correct, dim3(cell_blocks), dim3(256), 0, s, I.ctl.p, -1, MdfTest{}, I.cap, I.dptr.p,
@@ -2741,79 +2742,54 @@ uint64_t splitmix64_at(uint64_t seed, uint64_t k) {
 
 double splitmix64_unit(uint64_t seed, uint64_t k) { return (double)(splitmix64_at(seed, k) >> 11) * (1.0 / 9007199254740992.0); }
 
-int mlp_workspace(Mlp &M, int n) {
-  HIPCHK(M.H1.ensure((size_t)n * kMlpH));
-  HIPCHK(M.H2.ensure((size_t)n * kMlpH));
-  HIPCHK(M.H3.ensure((size_t)n * kMlpH));
-  HIPCHK(M.dZ3.ensure((size_t)n * kMlpH));
-  HIPCHK(M.dZ2.ensure((size_t)n * kMlpH));
-  HIPCHK(M.dZ1.ensure((size_t)n * kMlpH));
-  HIPCHK(M.Yp.ensure((size_t)n * kMlpOut));
-  HIPCHK(M.dY.ensure((size_t)n * kMlpOut));
-  HIPCHK(M.part.ensure(((size_t)n * kMlpOut + 255) / 256));
+// workgroups of k_mlp_rows for n rows: as many as share the 64-row tiles
+// evenly, at most kGradBlocks (one per CU: the kernel's LDS fills it)
+int mlp_blocks(int n) {
+  const int ntile = (n + kGradRows - 1) / kGradRows;
+  const int per = (ntile + kGradBlocks - 1) / kGradBlocks;
+  return (ntile + per - 1) / per;
+}
+
+// k_mlp_rows takes more dynamic LDS than the default limit
+template <bool GRAD>
+int mlp_rows_lds() {
+  static const hipError_t e = hipFuncSetAttribute((const void *)k_mlp_rows<GRAD>,
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpGradLds));
+  HIPCHK(e);
   return 0;
 }
 
-inline dim3 g256(long long n) { return dim3((unsigned)((n + 255) / 256)); }
-
-// FP32 forward of n samples into M.H1..H3, M.Yp
+// FP32 forward of n samples into M.Yp
 int mlp_forward32(Mlp &M, const float *X, int n) {
-  const float *th = M.th.p;
-  hipLaunchKernelGGL(k_dense_fwd, g256((long long)n * kMlpH), dim3(256), 0, M.s, X, n, kMlpIn, th + kMlpOffW1,
-                     th + kMlpOffB1, kMlpH, 1, M.H1.p);
-  hipLaunchKernelGGL(k_dense_fwd, g256((long long)n * kMlpH), dim3(256), 0, M.s, M.H1.p, n, kMlpH, th + kMlpOffW2,
-                     th + kMlpOffB2, kMlpH, 1, M.H2.p);
-  hipLaunchKernelGGL(k_dense_fwd, g256((long long)n * kMlpH), dim3(256), 0, M.s, M.H2.p, n, kMlpH, th + kMlpOffW3,
-                     th + kMlpOffB3, kMlpH, 1, M.H3.p);
-  hipLaunchKernelGGL(k_dense_fwd, g256((long long)n * kMlpOut), dim3(256), 0, M.s, M.H3.p, n, kMlpH,
-                     th + kMlpOffW4, th + kMlpOffB4, kMlpOut, 0, M.Yp.p);
+  if (mlp_rows_lds<false>()) return 1;
+  hipLaunchKernelGGL(k_mlp_rows<false>, dim3(mlp_blocks(n)), dim3(kGradThreads), sizeof(MlpGradLds), M.s, X, nullptr,
+                     nullptr, n, M.th.p, M.Yp.p, nullptr, nullptr);
   HIPCHK(hipGetLastError());
   return 0;
 }
 
-// forward + backward of n samples; gradient into M.g, squared-error block partials into M.part
-int mlp_fwd_bwd(Mlp &M, const float *X, const float *Y, int n) {
-  if (mlp_forward32(M, X, n)) return 1;
-  const float *th = M.th.p;
-  float *g = M.g.p;
-  const int cnt = n * kMlpOut;
-  hipLaunchKernelGGL(k_mse_grad, g256(cnt), dim3(256), 0, M.s, M.Yp.p, Y, cnt, M.dY.p, M.part.p);
-  hipLaunchKernelGGL(k_dense_bwd_w, g256(kMlpOut * kMlpH + kMlpOut), dim3(256), 0, M.s, M.dY.p, M.H3.p, n, kMlpOut,
-                     kMlpH, g + kMlpOffW4, g + kMlpOffB4);
-  hipLaunchKernelGGL(k_dense_bwd_in, g256((long long)n * kMlpH), dim3(256), 0, M.s, M.dY.p, n, kMlpOut,
-                     th + kMlpOffW4, kMlpH, M.H3.p, M.dZ3.p);
-  hipLaunchKernelGGL(k_dense_bwd_w, g256(kMlpH * kMlpH + kMlpH), dim3(256), 0, M.s, M.dZ3.p, M.H2.p, n, kMlpH,
-                     kMlpH, g + kMlpOffW3, g + kMlpOffB3);
-  hipLaunchKernelGGL(k_dense_bwd_in, g256((long long)n * kMlpH), dim3(256), 0, M.s, M.dZ3.p, n, kMlpH,
-                     th + kMlpOffW3, kMlpH, M.H2.p, M.dZ2.p);
-  hipLaunchKernelGGL(k_dense_bwd_w, g256(kMlpH * kMlpH + kMlpH), dim3(256), 0, M.s, M.dZ2.p, M.H1.p, n, kMlpH,
-                     kMlpH, g + kMlpOffW2, g + kMlpOffB2);
-  hipLaunchKernelGGL(k_dense_bwd_in, g256((long long)n * kMlpH), dim3(256), 0, M.s, M.dZ2.p, n, kMlpH,
-                     th + kMlpOffW2, kMlpH, M.H1.p, M.dZ1.p);
-  hipLaunchKernelGGL(k_dense_bwd_w, g256(kMlpH * kMlpIn + kMlpH), dim3(256), 0, M.s, M.dZ1.p, X, n, kMlpH, kMlpIn,
-                     g + kMlpOffW1, g + kMlpOffB1);
+// forward and backward of rows idx[0..n) (null: 0..n): the workgroups'
+// gradient parts into M.gpart, their squared errors into M.part
+int mlp_fwd_bwd(Mlp &M, const float *X, const float *Y, const int *idx, int n) {
+  if (mlp_rows_lds<true>()) return 1;
+  M.nblk = mlp_blocks(n);
+  HIPCHK(M.gpart.ensure((size_t)M.nblk * kMlpParams));
+  HIPCHK(M.part.ensure(M.nblk));
+  hipLaunchKernelGGL(k_mlp_rows<true>, dim3(M.nblk), dim3(kGradThreads), sizeof(MlpGradLds), M.s, X, Y, idx, n,
+                     M.th.p, nullptr, M.gpart.p, M.part.p);
   HIPCHK(hipGetLastError());
   return 0;
 }
 
 int mlp_loss(Mlp &M, int n, double *loss) {
-  const int cnt = n * kMlpOut, nb = (cnt + 255) / 256;
-  std::vector<double> p(nb);
-  HIPCHK(hipMemcpyAsync(p.data(), M.part.p, nb * sizeof(double), hipMemcpyDeviceToHost, M.s));
+  const int cnt = n * kMlpOut;
+  std::vector<double> p(M.nblk);
+  HIPCHK(hipMemcpyAsync(p.data(), M.part.p, M.nblk * sizeof(double), hipMemcpyDeviceToHost, M.s));
   HIPCHK(hipStreamSynchronize(M.s));
   double t = 0.0;
   for (double v : p) t = t + v;
   *loss = t / (double)cnt;
   return 0;
-}
-
-// rows idx[0..nb) of X/Y into the batch buffers
-__global__ void k_gather_rows(const float *__restrict__ src, const int *__restrict__ idx, int nb, int width,
-                              float *__restrict__ dst) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nb * width) return;
-  const int r = t / width, c = t - r * width;
-  dst[t] = src[(size_t)idx[r] * width + c];
 }
 
 }  // namespace
@@ -2879,9 +2855,9 @@ int fsil_mlp_forward(int handle, const float *X, int n, float *Y, int bf16) {
   if (n <= 0 || !X || !Y) return fail("bad arguments to fsil_mlp_forward");
   HIPCHK(M->X.ensure((size_t)n * kMlpIn));
   HIPCHK(hipMemcpyAsync(M->X.p, X, (size_t)n * kMlpIn * sizeof(float), hipMemcpyHostToDevice, M->s));
-  if (mlp_workspace(*M, n)) return 1;
+  HIPCHK(M->Yp.ensure((size_t)n * kMlpOut));
   if (bf16) {
-    hipLaunchKernelGGL(k_mlp_infer_bf16, dim3((n + 63) / 64), dim3(256), 0, M->s, M->X.p, n, M->th.p, M->Yp.p);
+    hipLaunchKernelGGL(k_mlp_infer_bf16, dim3(std::min(kInferBlocks, (n + 63) / 64)), dim3(256), 0, M->s, M->X.p, n, M->th.p, M->Yp.p);
     HIPCHK(hipGetLastError());
   } else {
     if (mlp_forward32(*M, M->X.p, n)) return 1;
@@ -2899,8 +2875,10 @@ int fsil_mlp_loss_grad(int handle, const float *X, const float *Y, int n, double
   HIPCHK(M->Y.ensure((size_t)n * kMlpOut));
   HIPCHK(hipMemcpyAsync(M->X.p, X, (size_t)n * kMlpIn * sizeof(float), hipMemcpyHostToDevice, M->s));
   HIPCHK(hipMemcpyAsync(M->Y.p, Y, (size_t)n * kMlpOut * sizeof(float), hipMemcpyHostToDevice, M->s));
-  if (mlp_workspace(*M, n)) return 1;
-  if (mlp_fwd_bwd(*M, M->X.p, M->Y.p, n)) return 1;
+  if (mlp_fwd_bwd(*M, M->X.p, M->Y.p, nullptr, n)) return 1;
+  hipLaunchKernelGGL(k_mlp_reduce<false>, dim3((kMlpParams + 63) / 64), dim3(256), 0, M->s, M->gpart.p, M->nblk,
+                     M->g.p, nullptr, nullptr, nullptr, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f);
+  HIPCHK(hipGetLastError());
   if (grad) HIPCHK(hipMemcpyAsync(grad, M->g.p, kMlpParams * sizeof(float), hipMemcpyDeviceToHost, M->s));
   double l = 0.0;
   if (mlp_loss(*M, n, &l)) return 1;
@@ -2916,14 +2894,11 @@ int fsil_mlp_train(int handle, const float *X, const float *Y, int n, int epochs
   batch = std::min(batch, n);
   HIPCHK(M->X.ensure((size_t)n * kMlpIn));
   HIPCHK(M->Y.ensure((size_t)n * kMlpOut));
-  HIPCHK(M->bx.ensure((size_t)batch * kMlpIn));
-  HIPCHK(M->by.ensure((size_t)batch * kMlpOut));
   HIPCHK(M->idx.ensure((size_t)n));
   HIPCHK(hipMemcpyAsync(M->X.p, X, (size_t)n * kMlpIn * sizeof(float), hipMemcpyHostToDevice, M->s));
   HIPCHK(hipMemcpyAsync(M->Y.p, Y, (size_t)n * kMlpOut * sizeof(float), hipMemcpyHostToDevice, M->s));
-  if (mlp_workspace(*M, std::max(n, batch))) return 1;
   if (loss_before) {
-    if (mlp_fwd_bwd(*M, M->X.p, M->Y.p, n)) return 1;
+    if (mlp_fwd_bwd(*M, M->X.p, M->Y.p, nullptr, n)) return 1;
     if (mlp_loss(*M, n, loss_before)) return 1;
   }
   std::vector<int> perm(n);
@@ -2937,20 +2912,16 @@ int fsil_mlp_train(int handle, const float *X, const float *Y, int n, int epochs
     HIPCHK(hipMemcpyAsync(M->idx.p, perm.data(), n * sizeof(int), hipMemcpyHostToDevice, M->s));
     HIPCHK(hipStreamSynchronize(M->s));  // perm is reused by the next epoch
     for (int b0 = 0; b0 + batch <= n; b0 += batch) {
-      hipLaunchKernelGGL(k_gather_rows, g256((long long)batch * kMlpIn), dim3(256), 0, M->s, M->X.p, M->idx.p + b0,
-                         batch, kMlpIn, M->bx.p);
-      hipLaunchKernelGGL(k_gather_rows, g256((long long)batch * kMlpOut), dim3(256), 0, M->s, M->Y.p,
-                         M->idx.p + b0, batch, kMlpOut, M->by.p);
-      if (mlp_fwd_bwd(*M, M->bx.p, M->by.p, batch)) return 1;
+      if (mlp_fwd_bwd(*M, M->X.p, M->Y.p, M->idx.p + b0, batch)) return 1;
       M->adam_t += 1;
       const float bc1 = 1.0f - std::pow(b1, (float)M->adam_t), bc2 = 1.0f - std::pow(b2, (float)M->adam_t);
-      hipLaunchKernelGGL(k_adam, g256(kMlpParams), dim3(256), 0, M->s, M->th.p, M->g.p, M->m.p, M->v.p, kMlpParams,
-                         (float)lr, b1, b2, eps, bc1, bc2);
+      hipLaunchKernelGGL(k_mlp_reduce<true>, dim3((kMlpParams + 63) / 64), dim3(256), 0, M->s, M->gpart.p, M->nblk,
+                         M->g.p, M->th.p, M->m.p, M->v.p, (float)lr, b1, b2, eps, bc1, bc2);
       HIPCHK(hipGetLastError());
     }
   }
   if (loss_after) {
-    if (mlp_fwd_bwd(*M, M->X.p, M->Y.p, n)) return 1;
+    if (mlp_fwd_bwd(*M, M->X.p, M->Y.p, nullptr, n)) return 1;
     if (mlp_loss(*M, n, loss_after)) return 1;
   }
   HIPCHK(hipStreamSynchronize(M->s));
