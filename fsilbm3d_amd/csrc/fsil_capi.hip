@@ -1051,18 +1051,25 @@ int fsil_block_create(int id, const int *dims, const double *geom, const int *bc
   if (iCollidModel == 3) {
     HIPCHK(b.Mc.ensure(Q * Q));
     HIPCHK(b.Mf.ensure(Q * Q));
-    HIPCHK(hipMemcpy(b.Mc.p, m_collid, Q * Q * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(b.Mf.p, m_force, Q * Q * sizeof(double), hipMemcpyHostToDevice));
+    // the device holds the matrices by rows (row_dot)
+    double mc[Q * Q], mf[Q * Q];
+    for (int i = 0; i < Q; ++i)
+      for (int j = 0; j < Q; ++j) {
+        mc[i * Q + j] = m_collid[j * Q + i];
+        mf[i * Q + j] = m_force[j * Q + i];
+      }
+    HIPCHK(hipMemcpy(b.Mc.p, mc, sizeof(mc), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(b.Mf.p, mf, sizeof(mf), hipMemcpyHostToDevice));
     if (precision == 1) {
-      float mc[Q * Q], mf[Q * Q];
+      float c32[Q * Q], f32[Q * Q];
       for (int k = 0; k < Q * Q; ++k) {
-        mc[k] = (float)m_collid[k];
-        mf[k] = (float)m_force[k];
+        c32[k] = (float)mc[k];
+        f32[k] = (float)mf[k];
       }
       HIPCHK(b.Mc32.ensure(Q * Q));
       HIPCHK(b.Mf32.ensure(Q * Q));
-      HIPCHK(hipMemcpy(b.Mc32.p, mc, sizeof(mc), hipMemcpyHostToDevice));
-      HIPCHK(hipMemcpy(b.Mf32.p, mf, sizeof(mf), hipMemcpyHostToDevice));
+      HIPCHK(hipMemcpy(b.Mc32.p, c32, sizeof(c32), hipMemcpyHostToDevice));
+      HIPCHK(hipMemcpy(b.Mf32.p, f32, sizeof(f32), hipMemcpyHostToDevice));
     }
   }
   for (int face = 0; face < 6; ++face) {

@@ -57,6 +57,26 @@ __device__ __forceinline__ unsigned voff(unsigned o) {
   return o;
 }
 
+// s + row . v in ascending order, row = 19 launch-uniform values read through
+// scalar registers.  The empty asm makes the row's reads wait for `after`, the
+// result of an earlier row: hoisted to the front of an unrolled 19 x 19
+// product the reads take more registers than there are (the kernels spilled
+// 160-1700 of them).  FP64 MRT with a volume force, 160x96x77 cells: 332 us
+// per launch with the spills, 123 us this way (its 2,900 FP64 operations per
+// cell take about 55 us, its 304 bytes 57 us).
+template <typename T> using cptr = __attribute__((address_space(4))) const T *;
+template <bool FMA, typename T>
+__device__ __forceinline__ T row_dot(const T *row, const T (&v)[Q], T s, T after) {
+  cptr<T> c = (cptr<T>)row;
+  asm volatile("" : "+s"(c) : "v"(after));
+#pragma unroll
+  for (int j = 0; j < Q; ++j) {
+    if constexpr (FMA) s = __builtin_fmaf(c[j], v[j], s);
+    else s = s + c[j] * v[j];
+  }
+  return s;
+}
+
 // The 19 values of one cell, v[q] = plane q at byte offset off.  nt streams
 // them past the caches (nontemporal); the choice is uniform over a launch.
 template <typename T>

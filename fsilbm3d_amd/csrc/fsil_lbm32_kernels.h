@@ -23,7 +23,7 @@ struct Collide32Args {
   long long N;
   float Omega, c1, dt3;
   float hO, hO2, cT1, cT2;                  // TRT: 0.5 Omega, 0.5 Omega2, 0.5 - 0.25 Omega, 0.5 - 0.25 Omega2
-  const float *__restrict__ Mc, *__restrict__ Mf;  // MRT: M_COLLID, M_FORCE rounded to FP32, column-major
+  const float *__restrict__ Mc, *__restrict__ Mf;  // MRT: M_COLLID, M_FORCE rounded to FP32, 19 rows of 19
   float hv[3];
   float VF[3];
   // immersed-boundary band overlay (corrected velocity and force, FP64)
@@ -105,10 +105,9 @@ __device__ __forceinline__ void moments32(const float *g, double &dr, double &j1
 // Guo term fl_q = 3 dh w_q (e_q.F (1 + 3 u.e_q) - u.F), the reference's
 // updates (FluidDomain.f90:1228-1238) read g'_q = g_q + (its f_q update);
 // fe of an opposite pair is w (A +- B) - g with the pair's A and B of the SRT
-// form.  MRT's matrices (rounded to FP32) are staged in LDS (ms, 2 x 361).
+// form.
 template <int MODEL, bool FORCE, bool BAND, bool NT>
-__device__ __forceinline__ void collide_push32_cell(const Collide32Args &a, int x, int y, int z, float *zx,
-                                                    const float *ms) {
+__device__ __forceinline__ void collide_push32_cell(const Collide32Args &a, int x, int y, int z, float *zx) {
   const unsigned n = ((unsigned)x * (unsigned)a.yd + (unsigned)y) * (unsigned)a.zd + (unsigned)z;
   const unsigned nb = n << 2;  // blocks of this form hold at most 2^30 cells
   const size_t plane = (size_t)a.N * sizeof(float);
@@ -198,13 +197,8 @@ __device__ __forceinline__ void collide_push32_cell(const Collide32Args &a, int 
       // MRT (FluidDomain.f90:1238): g + M_COLLID^T fe + M_FORCE^T fl
 #pragma unroll
       for (int i = 0; i < Q; ++i) {
-        float s = 0.0f;
-#pragma unroll
-        for (int j = 0; j < Q; ++j) s = __builtin_fmaf(ms[j * Q + i], fe[j], s);
-        if (forced) {
-#pragma unroll
-          for (int j = 0; j < Q; ++j) s = __builtin_fmaf(ms[Q * Q + j * Q + i], fl[j], s);
-        }
+        float s = row_dot<true>(a.Mc + i * Q, fe, 0.0f, i ? post[i - 1] : g[i]);
+        if (forced) s = row_dot<true>(a.Mf + i * Q, fl, s, s);
         post[i] = g[i] + s;
       }
     }
@@ -275,19 +269,9 @@ template <int MODEL, bool FORCE, bool BAND, bool NT>
 __global__ __launch_bounds__(512) void k_collide_push32(Collide32Args a) {
   // LDS of the exchange, sized at launch (zrow32_lds_bytes)
   extern __shared__ float zx[];
-  const float *ms = nullptr;
-  if constexpr (MODEL == 3) {
-    // the MRT matrices into LDS (every thread reads them in the same order: broadcasts)
-    __shared__ float mlds[2 * Q * Q];
-    const int nt = (int)(blockDim.x * blockDim.y);
-    for (int i = (int)(threadIdx.y * blockDim.x + threadIdx.x); i < 2 * Q * Q; i += nt)
-      mlds[i] = i < Q * Q ? a.Mc[i] : a.Mf[i - Q * Q];
-    __syncthreads();
-    ms = mlds;
-  }
   if (a.region == kRegionHull) {
     for_hull_cells(a.ctl, a.hole, a.xd, a.yd, a.zd, [&](int x, int y, int z) {
-      if (z < a.zd && y < a.yd) collide_push32_cell<MODEL, FORCE, BAND, NT>(a, x, y, z, zx, ms);
+      if (z < a.zd && y < a.yd) collide_push32_cell<MODEL, FORCE, BAND, NT>(a, x, y, z, zx);
     });
     return;
   }
@@ -296,7 +280,7 @@ __global__ __launch_bounds__(512) void k_collide_push32(Collide32Args a) {
   const int x = blockIdx.z;
   if (z >= a.zd || y >= a.yd) return;
   if (a.region == kRegionBulk && in_hole(a.hole, x, y)) return;
-  collide_push32_cell<MODEL, FORCE, BAND, NT>(a, x, y, z, zx, ms);
+  collide_push32_cell<MODEL, FORCE, BAND, NT>(a, x, y, z, zx);
 }
 
 // dynamic LDS of k_collide_push32 for its exchange mode and workgroup size

@@ -127,7 +127,7 @@ struct CollideArgs {
   double hO2, cT2;  // TRT: 0.5*Omega2, 0.5-0.25*Omega2
   double hv[3];     // 0.5*VF*dh   (numerator shift of the velocity moment)
   double VF[3];     // uniform volume force
-  const double *__restrict__ Mc;  // MRT M_COLLID, Fortran column-major 19x19
+  const double *__restrict__ Mc;  // MRT M_COLLID, 19 rows of 19
   const double *__restrict__ Mf;  // MRT M_FORCE
   // immersed-boundary band overlay (cells whose velocity/force come from IBM)
   const int *__restrict__ ctl;        // band bounding box in ctl[0..5] (device memory)
@@ -383,14 +383,8 @@ __device__ __forceinline__ void collide_push_cell(const CollideArgs &a, int x, i
     // MRT  (FluidDomain.f90:1238): f + MATMUL(M_COLLID,fEq) + MATMUL(M_FORCE,Flb)
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
-      double s = 0.0;
-      for (int j = 0; j < Q; ++j) s = s + a.Mc[j * Q + i] * fe[j];
-      double t = f[i] + s;
-      if (forced) {
-        double r = 0.0;
-        for (int j = 0; j < Q; ++j) r = r + a.Mf[j * Q + i] * fl[j];
-        t = t + r;
-      }
+      double t = f[i] + row_dot<false>(a.Mc + i * Q, fe, 0.0, i ? post[i - 1] : f[i]);
+      if (forced) t = t + row_dot<false>(a.Mf + i * Q, fl, 0.0, t);
       post[i] = t;
     }
   }
