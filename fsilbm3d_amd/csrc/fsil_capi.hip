@@ -2512,10 +2512,10 @@ int father_to_son(Block &F, Block &S, Pair &p, int n_timeStep) {
   for (int face = 0; face < 6; ++face)
     if (t.face[face].active) maxn = std::max(maxn, t.face[face].aS * t.face[face].bS);
   if (maxn == 0) return 0;
-  const dim3 grid((maxn + 255) / 256, 6);
+  const dim3 grid((maxn + kTreeNodes - 1) / kTreeNodes, 6), blk(kTreeNodes, Q);
   const int level = n_timeStep == 0 ? 1 : 2;
-  if (p.scheme == 2) hipLaunchKernelGGL(k_tree_father_to_son<2>, grid, dim3(256), 0, F.stream, t, level);
-  else hipLaunchKernelGGL(k_tree_father_to_son<1>, grid, dim3(256), 0, F.stream, t, level);
+  if (p.scheme == 2) hipLaunchKernelGGL(k_tree_father_to_son<2>, grid, blk, 0, F.stream, t, level);
+  else hipLaunchKernelGGL(k_tree_father_to_son<1>, grid, blk, 0, F.stream, t, level);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -2532,7 +2532,8 @@ int son_to_father(Block &F, Block &S, Pair &p) {
     maxn = std::max(maxn, t.sicnt[ea] * t.sicnt[eb]);
   }
   if (maxn == 0) return 0;
-  hipLaunchKernelGGL(k_tree_son_to_father, dim3((maxn + 255) / 256, 6), dim3(256), 0, F.stream, t);
+  hipLaunchKernelGGL(k_tree_son_to_father, dim3((maxn + kTreeNodes - 1) / kTreeNodes, 6), dim3(kTreeNodes, Q), 0, F.stream,
+                     t);
   HIPCHK(hipGetLastError());
   return 0;
 }
