@@ -493,66 +493,72 @@ int launch_faces(Block &b) {
   return 0;
 }
 
+// Workgroup of the cell kernels.  Rows of up to kCellThreads cells: whole
+// z-rows (the z-moving values are then exchanged inside the workgroup), as
+// many as fit 256 threads, and more where that raises the part of the waves'
+// lanes in use by over 7% (133-cell rows: three, 399 of 448 lanes, 360 us for
+// 301x149x133 FP64 where one row fills 133 of 192 and takes 397; below that
+// larger workgroups gain nothing or, with the block in the caches, lose:
+// 128x96x80 LES 55.0 us with four rows, 52.1 with three).  Longer rows are
+// cut into the width of 256, 192 or 128 that leaves the fewest idle lanes.
 dim3 cell_block(const Block &b) {
-  // one block spans whole z-rows where possible so the z-shifted stores of a
-  // row stay inside one workgroup (and one XCD's L2); longer rows are cut into
-  // the width of 256, 192 or 128 that leaves the fewest idle lanes
-  // (384-cell rows: two blocks of 192 rather than 256 + a half-idle 256)
-  int tz = b.zd;
-  if (b.zd > 256) {
+  if (b.zd <= kCellThreads) {
     int best = 0;
-    for (int w : {256, 192, 128}) {
-      const int lanes = (b.zd + w - 1) / w * w;
-      if (best == 0 || lanes < (b.zd + best - 1) / best * best) best = w;
+    double use = 0.0;
+    for (int ty = std::max(1, std::min(256 / b.zd, b.yd)); ty <= std::min(kCellThreads / b.zd, b.yd); ++ty) {
+      const int n = b.zd * ty;
+      const double u = (double)n / (double)((n + 63) / 64 * 64);
+      if (u > 1.07 * use) {
+        use = u;
+        best = ty;
+      }
     }
-    tz = best;
+    return dim3(b.zd, best, 1);
   }
-  int ty = std::max(1, 256 / tz);
-  ty = std::min(ty, b.yd);
-  return dim3(tz, ty, 1);
+  int tz = 0;
+  for (int w : {256, 192, 128}) {
+    const int lanes = (b.zd + w - 1) / w * w;
+    if (tz == 0 || lanes < (b.zd + tz - 1) / tz * tz) tz = w;
+  }
+  return dim3(tz, 1, 1);
 }
 
-// Workgroup of the FP32-deviation kernel (at most 512 threads, ~70 VGPRs):
-// rows of whole waves up to 512 cells are one workgroup (384-cell rows: six
-// waves, so the row exchange applies), else the shape of cell_block.
-dim3 cell_block32(const Block &b) {
-  if (b.zd > 256 && b.zd <= 512 && b.zd % 64 == 0) return dim3(b.zd, 1, 1);
-  return cell_block(b);
-}
-
-// The FP32-deviation kernel exchanges the z-moving values of a row through LDS when a
-// workgroup is whole z-rows and the grid has no idle threads (every thread
-// reaches the exchange's barrier); FSIL_ZROW=0 turns it off.  Resolved once at
-// block creation, so the launch and the cache policy agree.
+// The collide kernels exchange the z-moving values of a row inside the
+// workgroup when it is whole z-rows; FSIL_ZROW=0 turns it off.  Resolved once
+// at block creation, so the launch and the cache policy agree.
 int zrow_exchange(const Block &b, dim3 blk) {
   const char *e = getenv("FSIL_ZROW");
   if (e && !strcmp(e, "0")) return 0;
-  if (!((int)blk.x == b.zd && b.yd % (int)blk.y == 0 && blk.x * blk.y <= 512)) return 0;
-  // rows of whole waves: lane permutes, 320 bytes of LDS (FSIL_ZROW=1 forces the LDS form)
-  if (b.zd % 64 == 0 && !(e && !strcmp(e, "1"))) return 2;
+  if ((int)blk.x != b.zd) return 0;
+  // FP32 rows of whole waves: lane permutes, 80 bytes of LDS per wave (FSIL_ZROW=1 forces the LDS form)
+  if (b.precision == 1 && b.zd % 64 == 0 && !(e && !strcmp(e, "1"))) return 2;
   return 1;
 }
 
-// Cache policy of the fused kernel's population streams.  Measured on MI355X
-// (both storage forms, periodic blocks): plain loads and stores are 8-12%
-// faster at 384x192x192 and 512x256x256 (1-5 GB per population copy), where
-// the caches merge the partial lines of the z-shifted stores; nontemporal ones
-// are 3-14% faster at 1024x384x384 (11.5-23 GB per copy).  The switch is at
-// 8 GiB per copy.  FP32-deviation blocks whose workgroups are whole z-rows
-// store whole lines (zrow_exchange) and stream nontemporally at every size
-// (384x192x192: 5.49 TB/s against 5.22 plain; 512x256x256: 5.76 against
-// 5.43).  Blocks with coupled bodies always stream nontemporally
-// (stream_hint_for): there the beam solver runs beside the collide kernel and
-// the plain form's cache footprint slows the whole step (flexible plate,
-// 384x192x192: 0.92 -> 1.19 ms FP32-deviation, 1.24 -> 1.43 ms FP64, though
-// the collide kernel itself is 11% faster).  FSIL_STREAM_HINT=nt|plain
-// overrides the choice (at block creation) for tests that run both.
-int stream_policy(long long N, int precision, bool zrow) {
+// dynamic LDS of a collide launch for its exchange mode, workgroup and value size
+size_t zrow_lds_bytes(int zrow, dim3 blk, size_t value) {
+  const size_t threads = (size_t)blk.x * blk.y;
+  return zrow == 2 ? threads / 64 * 2 * 10 * value : (zrow == 1 ? 10 * threads * value : 0);
+}
+
+// Cache policy of the fused kernel's population streams.  Plain streams win
+// where the caches merge the partial lines that a launch stores: rows that
+// are not whole 128-byte lines (300x150x133 FP64: 399 us plain, 449
+// nontemporal), rows without the exchange up to 8 GiB per copy (384x192x192
+// FP64: 853 against 906; nontemporal is 3-14% faster above), and blocks whose
+// two copies stay in the 256 MB last-level cache (128x96x80 FP64, 299 MB: 49
+// against 54).  The rest, whole lines of larger blocks, streams nontemporally
+// (384x192x192 FP64: 788 against 808; 512x256x256: 1853 against 1929;
+// 200x120x64, 467 MB: 85.5 against 89.7; FP32 alike).
+// FSIL_STREAM_HINT=nt|plain overrides the choice (at block creation) for
+// tests that run both.
+int stream_policy(const Block &b) {
   const char *e = getenv("FSIL_STREAM_HINT");
   if (e && !strcmp(e, "nt")) return 1;
   if (e && !strcmp(e, "plain")) return 0;
-  if (precision == 1 && zrow) return 1;  // whole-line stores: nontemporal is faster at every size measured
-  const double copy_bytes = (double)Q * (double)N * (precision == 0 ? 8.0 : 4.0);
+  const size_t value = b.precision == 0 ? 8 : 4;
+  const double copy_bytes = (double)Q * (double)b.N * (double)value;
+  if (b.zrow && (size_t)b.zd * value % 128 == 0) return copy_bytes > 200.0e6 ? 1 : 0;
   return copy_bytes > 8.0 * 1024 * 1024 * 1024 ? 1 : 0;
 }
 
@@ -567,11 +573,11 @@ int stream_hint_for(const Block &b, bool band) {
 
 template <int MODEL>
 void launch_collide_model(const CollideArgs &a, bool force, bool band, bool aux, dim3 grid,
-                          dim3 blk, hipStream_t s) {
+                          dim3 blk, size_t lds, hipStream_t s) {
 #define L(F, B, X)                                                                                  \
   if (force == F && band == B && aux == X) {                                                        \
-    if (a.nt) hipLaunchKernelGGL((k_collide_push<MODEL, F, B, X, true>), grid, blk, 0, s, a);        \
-    else hipLaunchKernelGGL((k_collide_push<MODEL, F, B, X, false>), grid, blk, 0, s, a);            \
+    if (a.nt) hipLaunchKernelGGL((k_collide_push<MODEL, F, B, X, true>), grid, blk, lds, s, a);        \
+    else hipLaunchKernelGGL((k_collide_push<MODEL, F, B, X, false>), grid, blk, lds, s, a);            \
     return;                                                                                         \
   }
   L(false, false, false) L(true, false, false) L(false, true, false) L(true, true, false)
@@ -636,6 +642,8 @@ int collide_stream(Block &b, int region = kRegionAll, const int *hole = nullptr)
   const dim3 blk = cell_block(b);
   const dim3 grid = region == kRegionHull ? dim3(hull_grid(b, hole, blk))
                                           : dim3((b.zd + blk.x - 1) / blk.x, (b.yd + blk.y - 1) / blk.y, b.xd);
+  a.zrow = b.zrow;
+  const size_t lds = zrow_lds_bytes(a.zrow, blk, sizeof(double));
   if (is_les(b.model)) {
     a.tau_all = b.tau_all.p;
     a.uf = b.uf.p;
@@ -650,12 +658,12 @@ int collide_stream(Block &b, int region = kRegionAll, const int *hole = nullptr)
       HIPCHK(hipGetLastError());
     }
   }
-  if (b.model == 1) launch_collide_model<1>(a, force, band, aux, grid, blk, b.stream);
-  else if (b.model == 2) launch_collide_model<2>(a, force, band, aux, grid, blk, b.stream);
-  else if (b.model == 3) launch_collide_model<3>(a, force, band, aux, grid, blk, b.stream);
-  else if (b.model == 11) launch_collide_model<11>(a, force, band, aux, grid, blk, b.stream);
-  else if (b.model == 14) launch_collide_model<14>(a, force, band, aux, grid, blk, b.stream);
-  else launch_collide_model<15>(a, force, band, aux, grid, blk, b.stream);
+  if (b.model == 1) launch_collide_model<1>(a, force, band, aux, grid, blk, lds, b.stream);
+  else if (b.model == 2) launch_collide_model<2>(a, force, band, aux, grid, blk, lds, b.stream);
+  else if (b.model == 3) launch_collide_model<3>(a, force, band, aux, grid, blk, lds, b.stream);
+  else if (b.model == 11) launch_collide_model<11>(a, force, band, aux, grid, blk, lds, b.stream);
+  else if (b.model == 14) launch_collide_model<14>(a, force, band, aux, grid, blk, lds, b.stream);
+  else launch_collide_model<15>(a, force, band, aux, grid, blk, lds, b.stream);
   HIPCHK(hipGetLastError());
   if (region == kRegionBulk) return 0;  // the hull launch completes the step
   for (int face = 0; face < 6; ++face)
@@ -710,11 +718,11 @@ int collide_stream32(Block &b, int region = kRegionAll, const int *hole = nullpt
   }
   a.aux_face_mask102 = m102;
   a.aux_face_mask_hw = mhw;
-  const dim3 blk = cell_block32(b);
+  const dim3 blk = cell_block(b);
   const dim3 grid = region == kRegionHull ? dim3(hull_grid(b, hole, blk))
                                           : dim3((b.zd + blk.x - 1) / blk.x, (b.yd + blk.y - 1) / blk.y, b.xd);
   a.zrow = b.zrow;
-  size_t lds = zrow32_lds_bytes(a.zrow, blk.x * blk.y);
+  size_t lds = zrow_lds_bytes(a.zrow, blk, sizeof(float));
   if (region == kRegionBulk) lds = std::max(lds, b.bulk_lds);  // (the kernel reads only the first bytes)
 #define L32M(M, F, B)                                                                                  \
   if (a.nt) hipLaunchKernelGGL((k_collide_push32<M, F, B, true>), grid, blk, lds, b.stream, a);          \
@@ -994,8 +1002,8 @@ int fsil_block_create(int id, const int *dims, const double *geom, const int *bc
   b.model = iCollidModel;
   b.tau = relax[0]; b.Omega = relax[1]; b.Omega2 = relax[2];
   b.precision = precision;
-  b.zrow = precision == 1 ? zrow_exchange(b, cell_block32(b)) : 0;
-  b.nt = stream_policy(b.N, precision, b.zrow != 0);
+  b.zrow = zrow_exchange(b, cell_block(b));
+  b.nt = stream_policy(b);
   b.nt_forced = getenv("FSIL_STREAM_HINT") != nullptr;
   b.sh = std::make_shared<StreamHolder>();
   HIPCHK(hipStreamCreateWithFlags(&b.sh->s, hipStreamNonBlocking));
@@ -1896,7 +1904,7 @@ int collide_any(Block &b, int region, const int *hole) {
 bool split_hole(const Block &b, int *hole) {
   const Ibm &I = b.ibm;
   if (!b.split_ok || !I.have_box || I.M == 0 || is_les(b.model) || !b.fem.fs || !b.fem.fs->s) return false;
-  const int by = (int)(b.precision == 1 ? cell_block32(b) : cell_block(b)).y;
+  const int by = (int)cell_block(b).y;
   const int m = b.split_margin;
   const int x0 = std::max(0, I.box[0] - m), x1 = std::min(b.xd - 1, I.box[3] + m);
   int y0 = std::max(0, I.box[1] - m), y1 = std::min(b.yd - 1, I.box[4] + m);

@@ -130,8 +130,8 @@ __device__ __forceinline__ void store_cell(const T (&v)[Q], T *planes, size_t pl
   }
 }
 
-// Whole z-rows per workgroup (blockDim.x == zDim and every thread a cell of
-// the block): the ten values that move along z (e_z = +-1) are exchanged
+// Whole z-rows per workgroup (blockDim.x == zDim; every thread takes part):
+// the ten values that move along z (e_z = +-1) are exchanged
 // through LDS so that each thread stores, at its own z, the value arriving
 // there from z - e_z (periodic within the row).  A wave's stores then cover
 // whole cache lines instead of lines shifted by one value.  lds holds

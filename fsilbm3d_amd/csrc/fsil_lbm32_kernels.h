@@ -33,8 +33,8 @@ struct Collide32Args {
   const double *__restrict__ band_F;  // [3][cap]
   int cap;
   int nt;    // nontemporal population loads and stores (selects the kernel instantiation)
-  int zrow;  // workgroups are whole z-rows covering the block exactly: 1 shift_rows_z,
-             // 2 shift_rows_z_waves (rows of whole waves)
+  int zrow;  // workgroups are whole z-rows: 1 shift_rows_z, 2 shift_rows_z_waves (rows of
+             // whole waves)
   int region;   // CollideRegion
   int hole[4];  // kRegionBulk / kRegionHull: x0, x1, y0, y1
   // auxiliary planes of boundary codes 102 (den/u of the first interior
@@ -107,7 +107,7 @@ __device__ __forceinline__ void moments32(const float *g, double &dr, double &j1
 // fe of an opposite pair is w (A +- B) - g with the pair's A and B of the SRT
 // form.
 template <int MODEL, bool FORCE, bool BAND, bool NT>
-__device__ __forceinline__ void collide_push32_cell(const Collide32Args &a, int x, int y, int z, float *zx) {
+__device__ __forceinline__ void collide_push32_cell(const Collide32Args &a, int x, int y, int z, bool on, float *zx) {
   const unsigned n = ((unsigned)x * (unsigned)a.yd + (unsigned)y) * (unsigned)a.zd + (unsigned)z;
   const unsigned nb = n << 2;  // blocks of this form hold at most 2^30 cells
   const size_t plane = (size_t)a.N * sizeof(float);
@@ -144,7 +144,7 @@ __device__ __forceinline__ void collide_push32_cell(const Collide32Args &a, int 
       const int axis = face >> 1, hi = face & 1;
       const int c = axis == 0 ? x : (axis == 1 ? y : z);
       const int nd = axis == 0 ? a.xd : (axis == 1 ? a.yd : a.zd);
-      if (c == (hi ? nd - 2 : 1)) {
+      if (on && c == (hi ? nd - 2 : 1)) {
         const int p = face_plane_index(face, x, y, z, a.yd, a.zd);
         const int np = axis == 0 ? a.yd * a.zd : (axis == 1 ? a.xd * a.zd : a.xd * a.yd);
         a.nb_den[face][p] = 1.0 + dr64;
@@ -249,43 +249,43 @@ __device__ __forceinline__ void collide_push32_cell(const Collide32Args &a, int 
       const int axis = face >> 1, hi = face & 1;
       const int c = axis == 0 ? x : (axis == 1 ? y : z);
       const int nd = axis == 0 ? a.xd : (axis == 1 ? a.yd : a.zd);
-      if (c == (hi ? nd - 1 : 0)) {
+      if (on && c == (hi ? nd - 1 : 0)) {
         const int p = face_plane_index(face, x, y, z, a.yd, a.zd);
         const int np = axis == 0 ? a.yd * a.zd : (axis == 1 ? a.xd * a.zd : a.xd * a.yd);
         for (int q = 0; q < Q; ++q) a.hw[face][(long long)q * np + p] = (double)post[q] + wt(q);
       }
     }
   }
-  if (a.zrow == 2) shift_rows_z_waves(post, zx);
-  else if (a.zrow) shift_rows_z(post, zx);
+  if (a.zrow) {
+    if (a.zrow == 2) shift_rows_z_waves(post, zx);
+    else shift_rows_z(post, zx);
+    if (!on) return;
+  }
   const unsigned st[6] = {sxp, sxm, syp, sym, a.zrow ? 0u : szp, a.zrow ? 0u : szm};
   store_cell(post, a.gout, plane, n, st, NT);
 }
 
 // The z-row exchange has workgroup barriers: a workgroup of whole z-rows is
 // skipped or covered as a whole (the host aligns the hole's y-range to the
-// workgroup's rows, and a hull tile is a workgroup's shape inside the block).
+// workgroup's rows; rows past the block's last one take part idle).
 template <int MODEL, bool FORCE, bool BAND, bool NT>
-__global__ __launch_bounds__(512) void k_collide_push32(Collide32Args a) {
+__global__ __launch_bounds__(kCellThreads) void k_collide_push32(Collide32Args a) {
   // LDS of the exchange, sized at launch (zrow32_lds_bytes)
   extern __shared__ float zx[];
   if (a.region == kRegionHull) {
     for_hull_cells(a.ctl, a.hole, a.xd, a.yd, a.zd, [&](int x, int y, int z) {
-      if (z < a.zd && y < a.yd) collide_push32_cell<MODEL, FORCE, BAND, NT>(a, x, y, z, zx);
+      if (z < a.zd && (y < a.yd || a.zrow))
+        collide_push32_cell<MODEL, FORCE, BAND, NT>(a, x, min(y, a.yd - 1), z, y < a.yd, zx);
     });
     return;
   }
   const int z = blockIdx.x * blockDim.x + threadIdx.x;
   const int y = blockIdx.y * blockDim.y + threadIdx.y;
   const int x = blockIdx.z;
-  if (z >= a.zd || y >= a.yd) return;
-  if (a.region == kRegionBulk && in_hole(a.hole, x, y)) return;
-  collide_push32_cell<MODEL, FORCE, BAND, NT>(a, x, y, z, zx);
-}
-
-// dynamic LDS of k_collide_push32 for its exchange mode and workgroup size
-inline size_t zrow32_lds_bytes(int zrow, unsigned threads) {
-  return zrow == 2 ? (threads / 64) * 2 * 10 * sizeof(float) : (zrow == 1 ? 10 * (size_t)threads * sizeof(float) : 0);
+  if (z >= a.zd || (y >= a.yd && !a.zrow)) return;  // (a whole-row workgroup stays together for its exchange)
+  const int yc = min(y, a.yd - 1);
+  if (a.region == kRegionBulk && in_hole(a.hole, x, yc)) return;
+  collide_push32_cell<MODEL, FORCE, BAND, NT>(a, x, yc, z, y < a.yd, zx);
 }
 
 // den/u of the FP32-deviation state, in FP64 output arrays
