@@ -44,15 +44,18 @@ struct FemArrays {
 
 __device__ inline void fem_sync() { __syncthreads(); }
 
-// s + t[0] + t[1] + ... + t[n-1], in that order.  The terms are read in
+// t[0] + t[1] + ... + t[n-1] from +0, in that order.  The terms are read in
 // batches of sixteen into registers, the next batch while the current one is
 // added, so only the chain of additions is serial.  Every batch read is
 // unconditional (the last full batch is read once more, unused) so that the
 // wait before a batch's additions covers that batch alone and not the
-// prefetch behind it.
-__device__ inline double ordered_sum(double s, const double *t, int n) {
+// prefetch behind it.  (Sixteen terms read at once, one per lane, and
+// broadcast by v_mov_b64 row_newbcast take 7.8 ns per term against 4.1: the
+// moves issue between the additions.  Batches of eight, two ahead: 6.5.)
+__device__ inline double ordered_sum(const double *t, int n) {
   constexpr int B = 16;
   const int nb = n / B;
+  double s = 0.0;
   // drain every outstanding memory access first (generic accesses elsewhere
   // in the kernel count on the LDS counter too), so that inside the loop only
   // the in-order LDS reads are pending and a batch waits for itself alone
@@ -85,6 +88,16 @@ __device__ inline double ordered_sum(double s, const double *t, int n) {
   }
   for (int i = nb * B; i < n; ++i) s = s + t[i];
   return s;
+}
+
+// The thread's index, defined afresh where it is asked for.  The phases of the
+// Newton iteration take it so that nothing they derive from it is kept in
+// registers across the other phases (hoisted out of the iteration, those
+// values filled the register file and spilled in the CG).
+__device__ inline int fem_tid() {
+  int t = (int)threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
 }
 
 // The conjugate-gradient vectors of one body: in LDS when they fit (the usual
@@ -183,7 +196,7 @@ __device__ inline void fem_tree_sums(const double *t1, const double *t2, int n, 
   r2 = s2;
 }
 
-// sum of terms[0..n) in order by one thread (tree: fem_tree_sums), broadcast.
+// sum of terms[0..n) in order by one wave (tree: fem_tree_sums), broadcast.
 // The caller passes a block barrier before *shared is written again.
 __device__ inline double fem_serial_sum(const double *terms, int n, double *shared, int tree = 0) {
   if (tree) {
@@ -191,7 +204,10 @@ __device__ inline double fem_serial_sum(const double *terms, int n, double *shar
     fem_tree_sums(terms, nullptr, n, r1, r2);
     return r1;
   }
-  if (threadIdx.x == 0) *shared = ordered_sum(0.0, terms, n);
+  if (threadIdx.x < 64) {
+    const double s = ordered_sum(terms, n);
+    if (threadIdx.x == 0) *shared = s;
+  }
   fem_sync();
   return *shared;
 }
@@ -226,68 +242,28 @@ __device__ inline void fem_pair_sums(const double *prod, int cap, int n, double 
     fem_tree_sums(prod, prod + cap, n, r1, r2);
     return;
   }
-  if (threadIdx.x == 0) shared[0] = ordered_sum(0.0, prod, n);
-  else if (threadIdx.x == 64) shared[1] = ordered_sum(0.0, prod + cap, n);
+  if (threadIdx.x < 128) {
+    const int w = (int)threadIdx.x >> 6;
+    const double s = ordered_sum(prod + w * cap, n);
+    if ((threadIdx.x & 63) == 0) shared[w] = s;
+  }
   fem_sync();
   r1 = shared[0];
   r2 = shared[1];
 }
 
-// Dot products in DOF order, broadcast through LDS.  The products a_i*b_i
-// (each one rounding, as in the sequential loop) are formed by the whole
-// workgroup into LDS; one thread then adds them in order, so the serial part
-// is only the chain of additions.  fem_dot2 runs two such chains side by side
-// on two waves.
-__device__ inline void fem_dot_chunks(const double *a, const double *b, const double *c, const double *d, int n,
-                                      double *shared, double *stage, int cap, double &r1, double &r2, int tree = 0) {
-  if (tree) {
-    double s1 = 0.0, s2 = 0.0;
-    for (int base = 0; base < n; base += cap) {
-      const int m = min(cap, n - base);
-      for (int i = threadIdx.x; i < m; i += blockDim.x) {
-        stage[i] = a[base + i] * b[base + i];
-        if (c) stage[cap + i] = c[base + i] * d[base + i];
-      }
-      fem_sync();
-      double t1, t2;
-      fem_tree_sums(stage, c ? stage + cap : nullptr, m, t1, t2);
-      s1 = s1 + t1;
-      s2 = s2 + t2;
-      fem_sync();
-    }
-    r1 = s1;
-    r2 = s2;
-    return;
-  }
-  double s1 = 0.0, s2 = 0.0;
-  for (int base = 0; base < n; base += cap) {
-    const int m = min(cap, n - base);
-    for (int i = threadIdx.x; i < m; i += blockDim.x) {
-      stage[i] = a[base + i] * b[base + i];
-      if (c) stage[cap + i] = c[base + i] * d[base + i];
-    }
-    fem_sync();
-    if (threadIdx.x == 0) s1 = ordered_sum(s1, stage, m);
-    else if (c && threadIdx.x == 64) s2 = ordered_sum(s2, stage + cap, m);
-    fem_sync();
-  }
-  if (threadIdx.x == 0) shared[0] = s1;
-  if (threadIdx.x == 64) shared[1] = s2;
-  fem_sync();
-  r1 = shared[0];
-  r2 = shared[1];
-  fem_sync();
-}
-
-__device__ inline double fem_dot(const double *a, const double *b, int n, double *shared, double *stage, int cap) {
-  double r1, r2;
-  fem_dot_chunks(a, b, nullptr, nullptr, n, shared, stage, cap, r1, r2);
-  return r1;
-}
-
+// The dot products a.b and c.d, broadcast: the products (each one rounding, as
+// in the sequential loop) are formed by the whole workgroup into LDS (stage,
+// 2 n), then added in DOF order by two waves side by side.
 __device__ inline void fem_dot2(const double *a, const double *b, const double *c, const double *d, int n,
-                                double *shared, double *stage, int cap, double &r1, double &r2, int tree = 0) {
-  fem_dot_chunks(a, b, c, d, n, shared, stage, cap, r1, r2, tree);
+                                double *shared, double *stage, double &r1, double &r2, int tree = 0) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    stage[i] = a[i] * b[i];
+    stage[n + i] = c[i] * d[i];
+  }
+  fem_sync();
+  fem_pair_sums(stage, n, n, shared, r1, r2, tree);
+  fem_sync();
 }
 
 // v from the lane the DPP control selects (0 where it selects none or the
@@ -314,144 +290,199 @@ __device__ inline double wave_sum_dpp(double v) {
   return v;
 }
 
-// Row g of the element-by-element product A v (Beam_MatrixMultipy,
-// SolidSolver.f90:2035-2049, then LocToGlobal): each element product in
-// ascending k, the products added in the DOF's element order, as fem_matvec
-// forms them.  vk(d) gives v at the body's DOF d.
-template <class VK>
-__device__ inline double fem_row(const FemVecs &V, const CgLds &C, int g, VK &&vk) {
-  double y = 0.0;
-  for (int q = C.ptr[g]; q < C.ptr[g + 1]; ++q) {
-    const int ent = C.ent[q], e = ent / NED, i = ent - e * NED;
-    const int n0 = 6 * V.en[2 * e], n1 = 6 * V.en[2 * e + 1];
-    const double *cc = C.coef + (size_t)e * kCoefStride + i;
-    double s = 0.0;
-#pragma unroll
-    for (int k = 0; k < NED; ++k) s = s + cc[k * NED] * vk(k < 6 ? n0 + k : n1 + (k - 6));
-    y = y + s;
-  }
-  return y;
-}
+// The largest double whose (correctly rounded) square root is <= 1e-6: the
+// CG's test sqrt(r.r) <= 1e-6 without the square root.
+constexpr double kCgStop = 0x1.19799812dea11p-40;
 
-// CG_Solve (SolidSolver.f90:1949-2020) for the forms whose dot products are
-// summed in a tree (FP32-deviation blocks), with the CG state in LDS: three
-// workgroup barriers per iteration (after A p and p.Ap, after the x, r, z
-// updates and r.r, r.z, after the direction update).  DOFs are owned sixty
-// (ten whole nodes) per wave, so that a node's block-Jacobi row reads r of its
-// own wave; each owner forms its row of A p, its updates and its terms of the
-// dot products, which are summed within each wave by DPP (wave_sum_dpp) and
-// then over the waves in wave order.  (Forming p = z + beta p at every reader instead, which saves
-// the third barrier, measured 29 us per sub-step for the A p phase against
-// 17 us: the repeated reads cost more than the barrier.)  x holds xF on
-// entry; returns 2 on a breakdown (zero p.Ap or r.z), else 0; adds the
+// CG_Solve (SolidSolver.f90:1949-2020) with each DOF's state in registers: its
+// row of its first two element matrices (all there are at a node of an
+// unbranched beam; more are read from LDS), its block-Jacobi row, x, r, p, z
+// and A p.  DOFs are owned sixty (ten whole nodes) per wave, all of them at
+// once; only the search direction and, within a wave, the residual go through
+// LDS.
+//
+// Bound: the latency of one workgroup's dependent steps.  What an iteration
+// reads from LDS is the direction at its row's nodes (the rows, index lists
+// and vectors were read there on every iteration before: 3.3 us per iteration
+// of the flexible plate's 294 DOFs summed in a tree, 8.7 in DOF order, against
+// 1.7 and 4.6).
+//
+// TREE: dot products summed within each wave by DPP (wave_sum_dpp), then over
+// the waves in wave order, three barriers per iteration (the forms held to a
+// tolerance).  Else in DOF order: the terms go through LDS (stage) and one wave
+// adds them, r.r and r.z on waves of different SIMDs, two barriers
+// more; zeros pad the terms to whole batches of ordered_sum (a sum that starts
+// at +0 is the same with +0 added).  The rest is the same, sum for sum, as in
+// fem_matvec and fem_precond.
+//
+// V.x holds xF on entry (visible to the workgroup) and the solution on return,
+// V.r the load.  Returns 2 on a breakdown (zero p.Ap or r.z), else 0; adds the
 // iterations to cg_total.
-__device__ inline int fem_cg_fused(const FemArrays &A, const FemBodyDesc &D, const FemVecs &V, const CgLds &C,
-                                   int &cg_total) {
-  __shared__ double partA[16], partB[2][16];
-  const int nG = 6 * D.nND, g0 = D.goff;
-  const int nw = (int)blockDim.x >> 6, wv = (int)threadIdx.x >> 6, ln = (int)threadIdx.x & 63;
-  const int span = 60 * nw;
-  const double err = 1.0e-6;
-  auto zrow = [&](int g) {  // z_g = (M^-1 r)_g, block Jacobi
-    const int node = g / 6, i = g - node * 6;
-    const double *B = V.blk + (size_t)node * 36;
-    double sz = 0.0;
+constexpr int kRowElems = 2;
+__host__ __device__ inline int fem_pad16(int n) { return (n + 15) & ~15; }
+template <bool TREE>
+__device__ inline int fem_cg_rows(const FemBodyDesc &D, const FemVecs &V, const CgLds &C, double *stage,
+                                  int &cg_total) {
+  __shared__ double part[3][16];
+  const int nG = 6 * D.nND;
+  const int tid = fem_tid(), wv = tid >> 6, ln = tid & 63, nw = (nG + 59) / 60;
+  const int g = wv * 60 + ln;
+  const bool on = ln < 60 && g < nG;
+  const int node = on ? g / 6 : 0;
+  // the DOF's rows (zeros past its last element) and the nodes they read
+  double cc[kRowElems][NED], B[6], x = 0.0, r = 0.0, p = 0.0, z = 0.0, Ap = 0.0, xF = 0.0;
+  int nd[kRowElems][2];
+  const int q0 = on ? C.ptr[g] : 0, q1 = on ? C.ptr[g + 1] : 0;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) sz = sz + B[i * 6 + k] * V.r[6 * node + k];
-    return V.fixed[g] ? 0.0 : sz;
-  };
-  // r = lodEffe - A x (fixed DOFs 0), z = M^-1 r, r.r and r.z
-  double a1 = 0.0, a2 = 0.0;
-  for (int base = 0; base < nG; base += span) {
-    const int g = base + wv * 60 + ln;
-    const bool on = ln < 60 && g < nG;
-    if (on) {
-      const double y = fem_row(V, C, g, [&](int d) { return V.x[d]; });
-      V.r[g] = V.fixed[g] ? 0.0 : A.lodEffe[g0 + g] - y;
+  for (int j = 0; j < kRowElems; ++j) {
+    const bool have = q0 + j < q1;
+    const int ent = have ? C.ent[q0 + j] : 0, e = ent / NED, i = ent - e * NED;
+    nd[j][0] = 6 * V.en[2 * e];
+    nd[j][1] = 6 * V.en[2 * e + 1];
+    const double *c = C.coef + (size_t)e * kCoefStride + i;
+#pragma unroll
+    for (int k = 0; k < NED; ++k) cc[j][k] = have ? c[k * NED] : 0.0;
+  }
+  const bool fixed = on && V.fixed[g] != 0;
+  const int nP = fem_pad16(nG);
+  if (!TREE && tid < nP - nG) stage[nG + tid] = stage[nP + nG + tid] = 0.0;
+#pragma unroll
+  for (int k = 0; k < 6; ++k) B[k] = on ? V.blk[(size_t)node * 36 + (g - 6 * node) * 6 + k] : 0.0;
+  // this DOF's row of A v
+  auto row = [&](const double *v) {
+    double y = 0.0;
+#pragma unroll
+    for (int j = 0; j < kRowElems; ++j) {
+      double s = 0.0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const double2 *u = reinterpret_cast<const double2 *>(v + nd[j][h]);
+        const double2 a = u[0], b = u[1], c = u[2];
+        s = s + cc[j][6 * h] * a.x;
+        s = s + cc[j][6 * h + 1] * a.y;
+        s = s + cc[j][6 * h + 2] * b.x;
+        s = s + cc[j][6 * h + 3] * b.y;
+        s = s + cc[j][6 * h + 4] * c.x;
+        s = s + cc[j][6 * h + 5] * c.y;
+      }
+      y = y + s;
     }
+    for (int q = q0 + kRowElems; q < q1; ++q) {
+      const int ent = C.ent[q], e = ent / NED, i = ent - e * NED;
+      const double *c = C.coef + (size_t)e * kCoefStride + i, *u = v + 6 * V.en[2 * e], *w = v + 6 * V.en[2 * e + 1];
+      double s = 0.0;
+#pragma unroll
+      for (int k = 0; k < NED; ++k) s = s + c[k * NED] * (k < 6 ? u[k] : w[k - 6]);
+      y = y + s;
+    }
+    return y;
+  };
+  // z = M^-1 r from the node's residuals (all owned by this wave)
+  auto precond = [&]() {
+    if (on) V.r[g] = r;
     wave_sync();
     if (on) {
-      const double z = zrow(g), r = V.r[g];
-      V.z[g] = z;
-      a1 = a1 + r * r;
-      a2 = a2 + r * z;
+      const double2 *u = reinterpret_cast<const double2 *>(V.r + 6 * node);
+      const double2 a = u[0], b = u[1], c = u[2];
+      double s = 0.0;
+      s = s + B[0] * a.x;
+      s = s + B[1] * a.y;
+      s = s + B[2] * b.x;
+      s = s + B[3] * b.y;
+      s = s + B[4] * c.x;
+      s = s + B[5] * c.y;
+      z = fixed ? 0.0 : s;
     }
+  };
+  // sums of one or two terms per DOF, into every thread
+  auto sum1 = [&](double t) {
+    if constexpr (TREE) {
+      const double w = wave_sum_dpp(t);
+      if (ln == 63) part[0][wv] = w;
+      fem_sync();
+      double s = 0.0;
+      for (int k = 0; k < nw; ++k) s = s + part[0][k];
+      return s;
+    } else {
+      if (on) stage[g] = t;
+      fem_sync();
+      if (wv == 0) {
+        const double s = ordered_sum(stage, nP);
+        if (ln == 0) part[0][0] = s;
+      }
+      fem_sync();
+      return part[0][0];
+    }
+  };
+  auto sum2 = [&](double t1, double t2, double &s1, double &s2) {
+    if constexpr (TREE) {
+      const double w1 = wave_sum_dpp(t1), w2 = wave_sum_dpp(t2);
+      if (ln == 63) { part[1][wv] = w1; part[2][wv] = w2; }
+      fem_sync();
+      s1 = 0.0;
+      s2 = 0.0;
+      for (int k = 0; k < nw; ++k) { s1 = s1 + part[1][k]; s2 = s2 + part[2][k]; }
+    } else {
+      if (on) { stage[g] = t1; stage[nP + g] = t2; }
+      fem_sync();
+      if (wv < 2) {
+        const double s = ordered_sum(stage + wv * nP, nP);
+        if (ln == 0) part[1 + wv][0] = s;
+      }
+      fem_sync();
+      s1 = part[1][0];
+      s2 = part[2][0];
+    }
+  };
+  // r = load - A x (fixed DOFs 0), z = M^-1 r, p = z
+  if (on) {
+    x = V.x[g];
+    xF = V.xF[g];
+    const double y = row(V.x);
+    r = fixed ? 0.0 : V.r[g] - y;
   }
-  a1 = wave_sum_dpp(a1);
-  a2 = wave_sum_dpp(a2);
-  if (ln == 63) { partB[0][wv] = a1; partB[1][wv] = a2; }
-  fem_sync();
-  double rr = 0.0, rsold = 0.0;
-  for (int w = 0; w < nw; ++w) { rr = rr + partB[0][w]; rsold = rsold + partB[1][w]; }
-  double rn = sqrt(rr);
-  if (rn <= err) return 0;
+  wave_sync();  // (the wave's loads are read)
+  precond();
+  p = z;
+  if (on) V.p[g] = p;
+  double rr, rsold;
+  sum2(on ? r * r : 0.0, on ? r * z : 0.0, rr, rsold);
+  if (rr <= kCgStop) return 0;
   if (fabs(rsold) <= 1.0e-30) return 2;
-  bool first = true;
+  int status = 0;
   for (int it = 1; it <= 10000; ++it) {
     ++cg_total;
-    // p (z on the first iteration), A p with the fixed DOFs zeroed, p.Ap
-    auto pk = [&](int d) { return first ? V.z[d] : V.p[d]; };
-    double a = 0.0;
-    for (int base = 0; base < nG; base += span) {
-      const int g = base + wv * 60 + ln;
-      if (ln < 60 && g < nG) {
-        double y = fem_row(V, C, g, pk);
-        if (V.fixed[g]) y = 0.0;
-        V.Ap[g] = y;
-        const double pg = pk(g);
-        if (first) V.p[g] = pg;  // p = z (read as z by every other reader)
-        a = a + pg * y;
-      }
+    // A p with the fixed DOFs zeroed, p.Ap
+    if (on) {
+      Ap = row(V.p);
+      if (fixed) Ap = 0.0;
     }
-    a = wave_sum_dpp(a);
-    if (ln == 63) partA[wv] = a;
-    fem_sync();
-    double pAp = 0.0;
-    for (int w = 0; w < nw; ++w) pAp = pAp + partA[w];
-    if (fabs(pAp) <= 1.0e-30) return 2;
+    const double pAp = sum1(on ? p * Ap : 0.0);
+    if (fabs(pAp) <= 1.0e-30) { status = 2; break; }
     const double alpha = rsold / pAp;
-    // x, r update, z = M^-1 r, r.r and r.z
-    a1 = 0.0;
-    a2 = 0.0;
-    for (int base = 0; base < nG; base += span) {
-      const int g = base + wv * 60 + ln;
-      const bool on = ln < 60 && g < nG;
-      if (on) {
-        double xv = V.x[g] + alpha * V.p[g];
-        if (V.fixed[g]) xv = V.xF[g];
-        V.x[g] = xv;
-        double rv = V.r[g] - alpha * V.Ap[g];
-        if (V.fixed[g]) rv = 0.0;
-        V.r[g] = rv;
-      }
-      wave_sync();
-      if (on) {
-        const double z = zrow(g), r = V.r[g];
-        V.z[g] = z;
-        a1 = a1 + r * r;
-        a2 = a2 + r * z;
-      }
+    if (on) {
+      x = x + alpha * p;
+      if (fixed) x = xF;
+      r = r - alpha * Ap;
+      if (fixed) r = 0.0;
     }
-    a1 = wave_sum_dpp(a1);
-    a2 = wave_sum_dpp(a2);
-    if (ln == 63) { partB[0][wv] = a1; partB[1][wv] = a2; }
-    fem_sync();
-    double rsnew = 0.0;
-    rr = 0.0;
-    for (int w = 0; w < nw; ++w) { rr = rr + partB[0][w]; rsnew = rsnew + partB[1][w]; }
-    rn = sqrt(rr);
-    if (rn <= err) break;
-    if (fabs(rsold) <= 1.0e-30) return 2;
+    precond();
+    double rsnew;
+    sum2(on ? r * r : 0.0, on ? r * z : 0.0, rr, rsnew);
+    if (rr <= kCgStop) break;
+    if (fabs(rsold) <= 1.0e-30) { status = 2; break; }
     const double beta = rsnew / rsold;
-    for (int base = 0; base < nG; base += span) {
-      const int g = base + wv * 60 + ln;
-      if (ln < 60 && g < nG) V.p[g] = V.fixed[g] ? 0.0 : V.z[g] + beta * V.p[g];
+    if (on) {
+      p = z + beta * p;
+      if (fixed) p = 0.0;
+      V.p[g] = p;
     }
-    fem_sync();
-    first = false;
     rsold = rsnew;
+    fem_sync();
   }
-  return 0;
+  if (on) V.x[g] = x;
+  fem_sync();
+  return status;
 }
 
 // LDS of k_fem_substep, in doubles, behind one double of slack (fem_lds_base)
@@ -472,10 +503,18 @@ __host__ __device__ inline size_t fem_lds_bytes(int work, int vec_lds, int max_n
   return d * sizeof(double);
 }
 
+// offset of the CG's assembly lists in the work area, in doubles: behind the
+// staging area (2 nG) and the element products, and behind the two padded
+// staging areas of fem_cg_rows
+__host__ __device__ inline int fem_cg_lists(int nND, int nEL) {
+  const int a = 12 * nND + NED * nEL, b = 2 * fem_pad16(6 * nND);
+  return a > b ? a : b;
+}
+
 // work-area doubles the CG's assembly lists need for one body (cg_lds)
 __host__ __device__ inline size_t fem_cg_work(int nND, int nEL) {
   const size_t nG = 6 * (size_t)nND, nent = NED * (size_t)nEL;
-  return 2 * nG + nent + (nG + 1 + nent + 1) / 2;
+  return fem_cg_lists(nND, nEL) + (nG + 1 + nent + 1) / 2;
 }
 
 __device__ constexpr HotMap kHotMapD{};
@@ -554,10 +593,11 @@ __device__ inline void fem_rkr_block(ET &E, double *cl, const double *c, const F
 
 // One sub-step of one body by the whole workgroup.  HOT: the body's element
 // fields of the Newton iterations are in LDS (H, BeamHot per element), else
-// every element access goes to the global BeamElem array.
+// every element access goes to the global BeamElem array.  first: the launch's
+// first sub-step, which brings the index lists into LDS.
 template <bool HOT>
 __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int work, int vec_lds, int cg_lds,
-                                        int coef_off, BeamHot *H) {
+                                        int coef_off, BeamHot *H, bool first) {
   __shared__ double sh_val;
   __shared__ double sh_pair[2];
   __shared__ int sh_flag;
@@ -578,14 +618,15 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
     V.xF = V.blk + 36 * (size_t)nN;
     int *fx = reinterpret_cast<int *>(V.xF + nG);
     int *en = fx + nG;
-    for (int g = threadIdx.x; g < nG; g += blockDim.x) fx[g] = A.fixed[g0 + g];
-    for (int e = threadIdx.x; e < nE; e += blockDim.x) {
-      en[2 * e] = A.el[D.eoff + e].node0;
-      en[2 * e + 1] = A.el[D.eoff + e].node1;
+    if (first) {
+      for (int g = threadIdx.x; g < nG; g += blockDim.x) fx[g] = A.fixed[g0 + g];
+      for (int e = threadIdx.x; e < nE; e += blockDim.x) {
+        en[2 * e] = A.el[D.eoff + e].node0;
+        en[2 * e + 1] = A.el[D.eoff + e].node1;
+      }
     }
     V.fixed = fx;
     V.en = en;
-    fem_sync();
   } else {
     V.x = A.x + g0; V.r = A.r + g0; V.p = A.p + g0; V.z = A.z + g0; V.Ap = A.Ap + g0;
     V.blk = A.blk + (size_t)D.noff * 36;
@@ -622,6 +663,23 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
     if (threadIdx.x == 0) { D.newton_iters = 0; D.cg_iters = 0; D.status = 0; D.dnorm = 0.0; }
     return;
   }
+  // the body's assembly lists for the CG in LDS (behind the dot-product
+  // staging area [0, 2 nG) and the element products)
+  CgLds C{};
+  C.coef = coefL;
+  if (cg_lds) {
+    C.lbuf = lds + 2 * nG;
+    int *ip = reinterpret_cast<int *>(lds + fem_cg_lists(nN, nE));
+    int *ep = ip + nG + 1;
+    if (first) {
+      const int p0 = A.dof_ptr[g0], nent = A.dof_ptr[g0 + nG] - p0;
+      for (int g = threadIdx.x; g <= nG; g += blockDim.x) ip[g] = A.dof_ptr[g0 + g] - p0;
+      for (int k = threadIdx.x; k < nent; k += blockDim.x) ep[k] = (A.dof_e[p0 + k] - D.eoff) * NED + A.dof_i[p0 + k];
+    }
+    C.ptr = ip;
+    C.ent = ep;
+    C.on = true;
+  }
   const double *c = D.coeffs;
   // prescribed positions of this sub-step and InitDspVelAccATTimeT (SolidSolver.f90:1916-1930)
   for (int e = threadIdx.x; e < nE; e += blockDim.x) {
@@ -643,22 +701,6 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
   int cg_total = 0;
   int status = 0;
   double dnorm = 1.0;
-  // the body's assembly lists for the CG in LDS (behind the dot-product
-  // staging area [0, 2 nG) and the element products), once per sub-step
-  CgLds C{};
-  C.coef = coefL;
-  if (cg_lds) {
-    C.lbuf = lds + 2 * nG;
-    int *ip = reinterpret_cast<int *>(lds + 2 * nG + NED * nE);
-    const int p0 = A.dof_ptr[g0], nent = A.dof_ptr[g0 + nG] - p0;
-    int *ep = ip + nG + 1;
-    for (int g = threadIdx.x; g <= nG; g += blockDim.x) ip[g] = A.dof_ptr[g0 + g] - p0;
-    for (int k = threadIdx.x; k < nent; k += blockDim.x) ep[k] = (A.dof_e[p0 + k] - D.eoff) * NED + A.dof_i[p0 + k];
-    C.ptr = ip;
-    C.ent = ep;
-    C.on = true;
-    fem_sync();
-  }
   // UpdateMatrixANDLoad (SolidSolver.f90:1932-1947).  Per element: internal
   // force from the local stiffness, local geometric stiffness.
   auto stress_phase = [&](int t0, int step) {
@@ -676,7 +718,7 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
     // slots per block), so that the block's stiffness and geometric patterns
     // are known where the products are formed (fem_rkr_block)
     const int epad = (nE + 63) & ~63;
-    for (int t = threadIdx.x; t < 16 * epad; t += blockDim.x) {
+    for (int t = fem_tid(); t < 16 * epad; t += blockDim.x) {
       const int blk = t / epad, e = t - blk * epad;
       if (e >= nE) continue;
       auto &E = EL(e);
@@ -724,6 +766,7 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
       }
       A.lodInte[g0 + g] = li;
       A.lodEffe[g0 + g] = le;
+      V.r[g] = le;  // (the CG's load, where it keeps its vectors)
     }
   };
   for (iter = 1; iter <= D.ntolFEM; ++iter) {
@@ -738,7 +781,7 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
       // rotation (2, 6) and the axial force with the geometric-stiffness
       // scalars (3, 7); then the forces themselves on waves 0, 4.  The end
       // rotations wait in the dot-product staging area (free here).
-      const int w = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63, nw4 = (int)blockDim.x >> 8;
+      const int tid = fem_tid(), w = tid >> 6, lane = tid & 63, nw4 = (int)blockDim.x >> 8;
       double *rot_ab = lds;  // [e][6]: a, b
       for (int e = (w >> 2) * 64 + lane; e < nE; e += nw4 * 64) {
         auto &E = EL(e);
@@ -760,7 +803,7 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
         }
       fem_sync();
       matrices_phase();
-      assembly_phase((int)blockDim.x - 1 - (int)threadIdx.x, blockDim.x);
+      assembly_phase((int)blockDim.x - 1 - fem_tid(), blockDim.x);
       fem_sync();
     } else {
       stress_phase(threadIdx.x, blockDim.x);
@@ -773,70 +816,76 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
       fem_sync();
     }
     // CG_Solve (SolidSolver.f90:1949-2020), block-Jacobi preconditioner
-    for (int g = threadIdx.x; g < nG; g += blockDim.x) {
+    for (int g = fem_tid(); g < nG; g += blockDim.x) {
       const double xf = V.fixed[g] ? (iter == 1 ? A.vBC[g0 + g] : 0.0) : 0.0;
       V.xF[g] = xf;
       V.x[g] = xf;
     }
     // block-Jacobi preconditioner (SolidSolver.f90:1966-1975, Invert6x6
-    // :2234-2279): Gauss-Jordan on each node's 6x12 block with one lane per
-    // row holding its row in registers, ten nodes per wave (lanes 0..59).
-    // Row exchanges are kept as a permutation (pr: logical row -> the node's
-    // lane holding it, the same in the node's six lanes) instead of moving
-    // rows; pivot columns and the pivot row move between the node's lanes by
-    // shuffles.  Step i divides and eliminates only the columns later steps
-    // read (left-half columns after i, the whole right half): a column's
-    // values depend only on itself and the pivot column, and a left-half
-    // column is not read after its own step, so the inverse (the right half)
-    // and every pivot choice are the sequential routine's, operation for
-    // operation.
+    // :2234-2279): Gauss-Jordan on each node's 6x12 block, ten nodes per wave
+    // (lanes 0..59), a node's lane c holding column c of both halves.  A step
+    // needs the pivot column alone from another lane (six shuffles); every
+    // lane then finds the pivot, exchanges the two rows, and divides and
+    // eliminates its own two columns.  Left-half columns are not read after
+    // their own step, and a column's values depend only on itself and the
+    // pivot columns, so the inverse (the right half) and every pivot choice
+    // are the sequential routine's, operation for operation.  (With a lane
+    // per row instead, the pivot row and its shared-out quotients moved
+    // between lanes too, 29 shuffles a step: 5.6 us per solve with the
+    // vectors' set-up, against 3.4.)
     {
-      const int lane = (int)threadIdx.x & 63;
-      const int wv = (int)threadIdx.x >> 6, nw = (int)blockDim.x >> 6;
-      const int ln = lane / 6, row = lane - 6 * ln;
+      const int tid = fem_tid(), lane = tid & 63, wv = tid >> 6, nw = (int)blockDim.x >> 6;
+      const int ln = lane / 6, c6 = lane - 6 * ln;
       const int lbase = 6 * ln;
       for (int base = wv * 10; base < nN; base += nw * 10) {
         const int n = base + ln;
         const bool act = lane < 60 && n < nN;
-        double a[12];
+        double Lc[6], Rc[6];
+        int fx[6];
 #pragma unroll
-        for (int j = 0; j < 12; ++j) a[j] = 0.0;
-        int fxr = 0, fxc[6];
-#pragma unroll
-        for (int j = 0; j < 6; ++j) fxc[j] = 0;
+        for (int k = 0; k < 6; ++k) {
+          Lc[k] = 0.0;
+          Rc[k] = k == c6 ? 1.0 : 0.0;
+          fx[k] = 0;
+        }
         if (act) {
-          for (int k = A.node_ptr[D.noff + n]; k < A.node_ptr[D.noff + n + 1]; ++k) {
-            const int o = A.node_h[k] ? 6 : 0;
-            if (coefL) {
-              const double *cl = coefL + (A.node_e[k] - D.eoff) * kCoefStride;
+          if (coefL && C.on) {
+            // (a node's elements are those of its first DOF, in the same order)
+            for (int q = C.ptr[6 * n]; q < C.ptr[6 * n + 1]; ++q) {
+              const int ent = C.ent[q], e = ent / NED, o = ent - e * NED;
+              const double *cl = coefL + e * kCoefStride + (o + c6) * NED + o;
 #pragma unroll
-              for (int j = 0; j < 6; ++j) a[j] = a[j] + cl[(o + j) * NED + o + row];
-            } else {
-              const BeamElem &E = A.el[A.node_e[k]];
+              for (int k = 0; k < 6; ++k) Lc[k] = Lc[k] + cl[k];
+            }
+          } else {
+            for (int q = A.node_ptr[D.noff + n]; q < A.node_ptr[D.noff + n + 1]; ++q) {
+              const int o = A.node_h[q] ? 6 : 0;
+              if (coefL) {
+                const double *cl = coefL + (A.node_e[q] - D.eoff) * kCoefStride + (o + c6) * NED + o;
 #pragma unroll
-              for (int j = 0; j < 6; ++j) a[j] = a[j] + E.coef[(o + row) * NED + o + j];
+                for (int k = 0; k < 6; ++k) Lc[k] = Lc[k] + cl[k];
+              } else {
+                const BeamElem &E = A.el[A.node_e[q]];
+#pragma unroll
+                for (int k = 0; k < 6; ++k) Lc[k] = Lc[k] + E.coef[(o + k) * NED + o + c6];
+              }
             }
           }
 #pragma unroll
-          for (int j = 0; j < 6; ++j) fxc[j] = V.fixed[6 * n + j];
-          fxr = V.fixed[6 * n + row];
+          for (int k = 0; k < 6; ++k) fx[k] = V.fixed[6 * n + k];
+          const int fxc = V.fixed[6 * n + c6];
+          // fixed DOFs: their rows and columns zeroed, unit diagonal
+#pragma unroll
+          for (int k = 0; k < 6; ++k)
+            if (fx[k] || fxc) Lc[k] = k == c6 && fxc ? 1.0 : 0.0;
         }
-        // fixed DOFs: their rows and columns zeroed, unit diagonal
-#pragma unroll
-        for (int j = 0; j < 6; ++j)
-          if (fxr || fxc[j]) a[j] = (j == row && fxr) ? 1.0 : 0.0;
-#pragma unroll
-        for (int j = 0; j < 6; ++j) a[6 + j] = j == row ? 1.0 : 0.0;
         int bad = 0;
-        int pr[6];
-#pragma unroll
-        for (int k = 0; k < 6; ++k) pr[k] = k;
 #pragma unroll
         for (int i = 0; i < 6; ++i) {
-          // column i of the node's logical rows, pivot as the sequential search picks it
+          // column i; the pivot as the sequential search picks it
           double col[6];
 #pragma unroll
-          for (int k = i; k < 6; ++k) col[k] = __shfl(a[i], lbase + pr[k], 64);
+          for (int k = 0; k < 6; ++k) col[k] = __shfl(Lc[k], lbase + i, 64);
           int p = i;
           double pivot = fabs(col[i]);
 #pragma unroll
@@ -846,70 +895,44 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
               p = k;
             }
           if (!bad && pivot <= 1.0e-30) bad = i + 1;
-          // logical rows i and p exchanged
+          // rows i and p exchanged (skipped where no node of the wave does)
+          if (__ballot(!bad && p != i)) {
+#pragma unroll
+            for (int k = i + 1; k < 6; ++k) {
+              const bool sw = !bad && k == p;
+              const double l = Lc[k], rt = Rc[k], cv = col[k];
+              Lc[k] = sw ? Lc[i] : l;
+              Lc[i] = sw ? l : Lc[i];
+              Rc[k] = sw ? Rc[i] : rt;
+              Rc[i] = sw ? rt : Rc[i];
+              col[k] = sw ? col[i] : cv;
+              col[i] = sw ? cv : col[i];
+            }
+          }
           if (!bad) {
-            const int pi = pr[i];
-            int pp = pi;
+            Lc[i] = Lc[i] / col[i];
+            Rc[i] = Rc[i] / col[i];
 #pragma unroll
-            for (int k = i + 1; k < 6; ++k)
-              if (k == p) pp = pr[k];
-#pragma unroll
-            for (int k = i + 1; k < 6; ++k)
-              if (k == p) pr[k] = pi;
-            pr[i] = pp;
-          }
-          const int P = pr[i];  // the node's lane holding the pivot row
-          // the pivot row divided by the pivot: the 11 - i quotients are
-          // shared out over the node's six lanes (two divisions per lane
-          // instead of 11 - i by the pivot's lane, whose divisions the whole
-          // wave would issue), then gathered by every lane
-          const double pv = __shfl(a[i], lbase + P, 64);
-          double raw[12];
-#pragma unroll
-          for (int j = i + 1; j < 12; ++j) raw[j] = __shfl(a[j], lbase + P, 64);
-          double n0 = 0.0, n1 = 0.0;
-#pragma unroll
-          for (int kk = 0; kk < 6; ++kk) {
-            if (row == kk && i + 1 + kk < 12) n0 = raw[i + 1 + kk];
-            if (row == kk && i + 7 + kk < 12) n1 = raw[i + 7 + kk];
-          }
-          double q0 = 0.0, q1 = 0.0;
-          if (!bad) {
-            q0 = n0 / pv;
-            q1 = n1 / pv;
-          }
-          double prow[12];
-#pragma unroll
-          for (int j = i + 1; j < 12; ++j) {
-            const int kk = j - i - 1;
-            prow[j] = kk < 6 ? __shfl(q0, lbase + kk, 64) : __shfl(q1, lbase + kk - 6, 64);
-          }
-          if (!bad && row == P) {
-#pragma unroll
-            for (int j = i + 1; j < 12; ++j) a[j] = prow[j];
-          }
-          if (!bad && row != P) {
-            const double factor = a[i];
-#pragma unroll
-            for (int j = i + 1; j < 12; ++j) a[j] = a[j] - factor * prow[j];
+            for (int k = 0; k < 6; ++k)
+              if (k != i) {
+                Lc[k] = Lc[k] - col[k] * Lc[i];
+                Rc[k] = Rc[k] - col[k] * Rc[i];
+              }
           }
         }
-        // this lane's logical row
-        int L = 0;
-#pragma unroll
-        for (int k = 0; k < 6; ++k)
-          if (pr[k] == row) L = k;
         if (act) {
           double *out = V.blk + (size_t)n * 36;
-          // (a singular block leaves the identity; pr is then still the start)
+          // (a singular block leaves the identity)
 #pragma unroll
-          for (int j = 0; j < 6; ++j) out[L * 6 + j] = bad ? (L == j ? 1.0 : 0.0) : a[6 + j];
+          for (int k = 0; k < 6; ++k) out[k * 6 + c6] = bad ? (k == c6 ? 1.0 : 0.0) : Rc[k];
         }
       }
     }
     fem_sync();
-    if (D.tree_sums && C.on && C.coef && V.en) {
-      if (const int st = fem_cg_fused(A, D, V, C, cg_total)) { status = st; break; }
+    if (nG <= 60 * ((int)blockDim.x >> 6) && C.on && C.coef && V.en) {
+      const int st = D.tree_sums ? fem_cg_rows<true>(D, V, C, lds, cg_total)
+                                 : fem_cg_rows<false>(D, V, C, lds, cg_total);
+      if (st) { status = st; break; }
     } else {
     fem_matvec(A, D, V, C, V.x, V.Ap);
     for (int g = threadIdx.x; g < nG; g += blockDim.x)
@@ -919,7 +942,7 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
     const double err = 1.0e-6;
     const int cap = nG;  // product staging: [0, nG) and [nG, 2 nG)
     double rr, rz;
-    fem_dot2(V.r, V.r, V.r, V.z, nG, sh_pair, lds, cap, rr, rz, D.tree_sums);
+    fem_dot2(V.r, V.r, V.r, V.z, nG, sh_pair, lds, rr, rz, D.tree_sums);
     double rn = sqrt(rr);
     if (!(rn <= err)) {
       for (int g = threadIdx.x; g < nG; g += blockDim.x) V.p[g] = V.z[g];
@@ -988,7 +1011,7 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
     // does not depend on the order; each wave's maximum goes to lds[wave]
     {
       double mx = -INFINITY;
-      for (int g = threadIdx.x; g < nG; g += blockDim.x) {
+      for (int g = fem_tid(); g < nG; g += blockDim.x) {
         A.dsp[g0 + g] = A.dsp[g0 + g] + V.x[g];
         const double v = V.x[g] * V.x[g];
         if (v > mx) mx = v;
@@ -1004,7 +1027,7 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
     // end and the current geometry; odd waves: the second end), then the
     // element triad
     {
-      const int w = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63, nw2 = (int)blockDim.x >> 7;
+      const int tid = fem_tid(), w = tid >> 6, lane = tid & 63, nw2 = (int)blockDim.x >> 7;
       for (int e = (w >> 1) * 64 + lane; e < nE; e += nw2 * 64) {
         auto &E = EL(e);
         if ((w & 1) == 0) {
@@ -1021,7 +1044,14 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
       }
     }
     fem_sync();
-    for (int e = threadIdx.x; e < nE; e += blockDim.x) el_make_triad_ee(EL(e));
+    for (int e = fem_tid(); e < nE; e += blockDim.x) el_make_triad_ee(EL(e));
+    // the node positions beside the element triads (from the top thread down)
+    for (int n = (int)blockDim.x - 1 - fem_tid(); n < nN; n += blockDim.x) {
+      const int last = A.node_ptr[D.noff + n + 1] - 1;
+      const auto &E = EL(A.node_e[last] - D.eoff);
+      const double *src = A.node_h[last] ? E.x1 + 6 : E.x1;
+      for (int k = 0; k < 6; ++k) A.pos[g0 + 6 * n + k] = src[k];
+    }
     {
       double m = lds[0];
       for (int w = 1; w < (int)(blockDim.x + 63) / 64; ++w)
@@ -1029,13 +1059,6 @@ __device__ inline void fem_substep_body(FemBodyDesc &D, const FemArrays &A, int 
       dnorm = fabs(m);
     }
     fem_sync();
-    // (nothing before the next rewrite of lds[0..waves) reads pos)
-    for (int n = threadIdx.x; n < nN; n += blockDim.x) {
-      const int last = A.node_ptr[D.noff + n + 1] - 1;
-      const auto &E = EL(A.node_e[last] - D.eoff);
-      const double *src = A.node_h[last] ? E.x1 + 6 : E.x1;
-      for (int k = 0; k < 6; ++k) A.pos[g0 + 6 * n + k] = src[k];
-    }
     if (dnorm <= D.dtolFEM) break;
   }
   // UpdateVelAcc (SolidSolver.f90:2350-2359)
@@ -1076,10 +1099,18 @@ __global__ __launch_bounds__(512) void k_fem_substep(FemBodyDesc *descs, int nbo
   BeamHot *H = HOT ? reinterpret_cast<BeamHot *>(lds + hot_off) : nullptr;
   long long *hw = reinterpret_cast<long long *>(H);
   bool hot = false;
+  // (each descriptor is read across the host link during the sub-step before)
+  constexpr int kDescWords = (int)(sizeof(FemBodyDesc) / 8);
+  auto desc = [&](int isub) { return descs + (size_t)isub * nbodies + blockIdx.x; };
+  auto word = [&](int isub) {
+    return isub < nsub && (int)threadIdx.x < kDescWords ? reinterpret_cast<const long long *>(desc(isub))[threadIdx.x]
+                                                        : 0LL;
+  };
+  long long next = word(0);
   for (int isub = 0; isub < nsub; ++isub) {
-    FemBodyDesc *g = descs + (size_t)isub * nbodies + blockIdx.x;
-    if (threadIdx.x < sizeof(FemBodyDesc) / 8)
-      reinterpret_cast<long long *>(&sD)[threadIdx.x] = reinterpret_cast<const long long *>(g)[threadIdx.x];
+    FemBodyDesc *g = desc(isub);
+    if ((int)threadIdx.x < kDescWords) reinterpret_cast<long long *>(&sD)[threadIdx.x] = next;
+    next = word(isub + 1);
     fem_sync();
     if constexpr (HOT) {
       if (isub == 0 && sD.iBodyModel != 1) {
@@ -1093,7 +1124,7 @@ __global__ __launch_bounds__(512) void k_fem_substep(FemBodyDesc *descs, int nbo
       }
     }
     // (a rigid body's sub-step does not reach the element fields)
-    fem_substep_body<HOT>(sD, A, work, vec_lds, cg_lds, coef_off, H);
+    fem_substep_body<HOT>(sD, A, work, vec_lds, cg_lds, coef_off, H, isub == 0);
     fem_sync();
     if (threadIdx.x == 0) {
       g->newton_iters = sD.newton_iters;
