@@ -282,7 +282,7 @@ struct Block {
   bool split = false;             // the coupling's launches go to the beam stream
   bool split_ok = true;           // FSIL_SPLIT=0 turns split steps off
   int split_margin = 3;           // cells the predicted band box adds to the last one (FSIL_SPLIT_MARGIN)
-  size_t bulk_lds = 0;            // dynamic LDS of an FP32 split step's bulk launch (its CU residency)
+  size_t bulk_lds = 0;            // dynamic LDS of a split step's bulk launch (its CU residency)
 };
 
 std::map<int, std::unique_ptr<Block>> g_blocks;
@@ -643,7 +643,8 @@ int collide_stream(Block &b, int region = kRegionAll, const int *hole = nullptr)
   const dim3 grid = region == kRegionHull ? dim3(hull_grid(b, hole, blk))
                                           : dim3((b.zd + blk.x - 1) / blk.x, (b.yd + blk.y - 1) / blk.y, b.xd);
   a.zrow = b.zrow;
-  const size_t lds = zrow_lds_bytes(a.zrow, blk, sizeof(double));
+  size_t lds = zrow_lds_bytes(a.zrow, blk, sizeof(double));
+  if (region == kRegionBulk) lds = std::max(lds, b.bulk_lds);  // (the kernel uses only the exchange's)
   if (is_les(b.model)) {
     a.tau_all = b.tau_all.p;
     a.uf = b.uf.p;
@@ -1012,22 +1013,20 @@ int fsil_block_create(int id, const int *dims, const double *geom, const int *bc
   HIPCHK(hipEventCreate(&b.ev1));
   HIPCHK(hipEventCreateWithFlags(&b.ev_fluid, hipEventDisableTiming));
   {
-    // Split steps pay where the coupling and beam chain is the step's critical
-    // path (FP32-deviation: 0.781 against 0.807 ms); in FP64 the fluid update
-    // is, and the split costs (flexible plate 1.174 against 1.152 ms):
+    // Split steps run the bulk of the collision beside the coupling call and
+    // the beam sub-steps (flexible plate 384x192x192, thirty steps and the
+    // flow output: FP64 31 ms against 38 unsplit; small blocks gain 3-10%);
     // FSIL_SPLIT=1 or 0 overrides.
     const char *e = getenv("FSIL_SPLIT");
-    b.split_ok = e ? strcmp(e, "0") != 0 : precision == 1;
+    b.split_ok = e ? strcmp(e, "0") != 0 : true;
     const char *m = getenv("FSIL_SPLIT_MARGIN");
     if (m) b.split_margin = atoi(m);
-    // The bulk launch of an FP32 split step runs beside the coupling call,
-    // whose small launches wait for CU slots while the bulk's workgroups fill
-    // every CU.  The bulk asks for enough LDS that at most R of its
-    // workgroups share a CU (FSIL_BULK_RESIDENCY=R, default 2; 0: no limit).
-    // Measured on MI355X, flexible plate 384x192x192: 0.714 ms per step
-    // unlimited (6 per CU), 0.689 at 4, 0.685 at 3, 0.675 at 2; the bulk
-    // itself takes 489 us at 2 against 405 us, the coupling's band build
-    // 57 us against 200 us.
+    // The coupling's small launches and the beam's workgroups wait for CU
+    // slots while the bulk's workgroups fill every CU.  The bulk asks for
+    // enough LDS that at most R of its workgroups share a CU
+    // (FSIL_BULK_RESIDENCY=R, default 2; 0: no limit).  Measured, ms for the
+    // same run at R = 2, 3, 4, 5: FP64 31.0, 31.2, 32.4, 33.7; sixty steps in
+    // FP32-deviation form 37.1, 37.2, 39.2, 40.0.
     int R = 2;
     if (const char *r = getenv("FSIL_BULK_RESIDENCY")) R = atoi(r);
     int dev = 0, per_cu = 0;
