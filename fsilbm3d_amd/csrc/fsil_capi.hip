@@ -251,7 +251,8 @@ struct Block {
   int precision = 0;  // 0 FP64 plain, 1 FP32 deviation storage
   int nt = 0;         // population streams nontemporal (see stream_policy)
   int zrow = 0;       // FP32 row exchange of the z-moving values (zrow_exchange), fixed at creation
-  bool nt_forced = false;  // FSIL_STREAM_HINT set at creation
+  ZFaces zf{};             // z faces that the collide launches apply
+  bool rim = false;        // the other faces take one launch (k_rim)
   DevBuf<double> fA, fB;
   DevBuf<float> gA, gB;
   DevBuf<double> Mc, Mf;
@@ -424,7 +425,9 @@ bool is_active_face(int code) {
   return !(code == BC_PERIODIC || code == BC_FLUID || code == BC_FLUID_FATHER);
 }
 
-int launch_faces(Block &b) {
+// The faces after a collide launch (after_collide: those that it has not
+// applied itself), or all of them.
+int launch_faces(Block &b, bool after_collide) {
   auto args = [&](int face) {
     FaceArgs a{};
     const int code = b.bc[face];
@@ -447,6 +450,21 @@ int launch_faces(Block &b) {
     a.hw = b.hw_valid[face] ? b.hw[face].p : nullptr;
     return a;
   };
+  if (after_collide && b.rim) {
+    RimArgs r{};
+    for (int face = 0; face < 6; ++face) {
+      r.f[face] = args(face);
+      if (is_active_face(b.bc[face])) r.active |= 1 << face;
+    }
+    const int nx = (r.active & 1) + ((r.active >> 1) & 1), ny = ((r.active >> 2) & 1) + ((r.active >> 3) & 1);
+    const int nodes = nx * b.yd * b.zd + ny * (b.xd - nx) * b.zd;
+    if (nodes == 0) return 0;
+    const dim3 grid((nodes + 255) / 256);
+    if (b.precision) hipLaunchKernelGGL(k_rim<true>, grid, dim3(256), 0, b.stream, r);
+    else hipLaunchKernelGGL(k_rim<false>, grid, dim3(256), 0, b.stream, r);
+    HIPCHK(hipGetLastError());
+    return 0;
+  }
   const dim3 block(256);
   const bool f32 = b.precision != 0;
   for (int axis = 0; axis < 3; ++axis) {
@@ -533,6 +551,30 @@ int zrow_exchange(const Block &b, dim3 blk) {
   // FP32 rows of whole waves: lane permutes, 80 bytes of LDS per wave (FSIL_ZROW=1 forces the LDS form)
   if (b.precision == 1 && b.zd % 64 == 0 && !(e && !strcmp(e, "1"))) return 2;
   return 1;
+}
+
+// Which faces the collide launches apply and whether the rest take one launch
+// (k_rim).  z faces that set a population from one arriving at the same node
+// (symmetry, wall) or from the node's own post-collision value (halfway wall)
+// are applied where the row exchange has those values at hand; k_rim needs the
+// y faces' codes to set a node from its own populations too.  Other
+// combinations, and blocks without whole-row workgroups, keep a launch per
+// axis.  FSIL_FACES=0 turns it off (at block creation) for tests that run both.
+void face_plan(Block &b) {
+  const char *e = getenv("FSIL_FACES");
+  if ((e && !strcmp(e, "0")) || !b.zrow || b.xd < 6 || b.yd < 6 || b.zd < 6) return;
+  for (int face = 2; face < 6; ++face) {
+    const int c = b.bc[face];
+    if (!is_active_face(c) || c == BC_SYMMETRIC || c == BC_WALL || c == BC_WALL_HALFWAY) continue;
+    if (face < 4 && (c == BC_EQ_DIRICHLET || c == BC_MOVING_WALL || c == BC_MOVING_WALL_HALFWAY)) continue;
+    return;
+  }
+  b.rim = true;
+  for (int face = 0; face < 6; ++face) {
+    if (!is_active_face(b.bc[face])) continue;
+    if (face < 4) b.zf.rim |= 1 << face;
+    else b.zf.code[face - 4] = b.bc[face];
+  }
 }
 
 // dynamic LDS of a collide launch for its exchange mode, workgroup and value size
@@ -643,6 +685,7 @@ int collide_stream(Block &b, int region = kRegionAll, const int *hole = nullptr)
   const dim3 grid = region == kRegionHull ? dim3(hull_grid(b, hole, blk))
                                           : dim3((b.zd + blk.x - 1) / blk.x, (b.yd + blk.y - 1) / blk.y, b.xd);
   a.zrow = b.zrow;
+  a.zf = b.zf;
   size_t lds = zrow_lds_bytes(a.zrow, blk, sizeof(double));
   if (region == kRegionBulk) lds = std::max(lds, b.bulk_lds);  // (the kernel uses only the exchange's)
   if (is_les(b.model)) {
@@ -723,6 +766,7 @@ int collide_stream32(Block &b, int region = kRegionAll, const int *hole = nullpt
   const dim3 grid = region == kRegionHull ? dim3(hull_grid(b, hole, blk))
                                           : dim3((b.zd + blk.x - 1) / blk.x, (b.yd + blk.y - 1) / blk.y, b.xd);
   a.zrow = b.zrow;
+  a.zf = b.zf;
   size_t lds = zrow_lds_bytes(a.zrow, blk, sizeof(float));
   if (region == kRegionBulk) lds = std::max(lds, b.bulk_lds);  // (the kernel reads only the first bytes)
 #define L32M(M, F, B)                                                                                  \
@@ -1005,7 +1049,7 @@ int fsil_block_create(int id, const int *dims, const double *geom, const int *bc
   b.precision = precision;
   b.zrow = zrow_exchange(b, cell_block(b));
   b.nt = stream_policy(b);
-  b.nt_forced = getenv("FSIL_STREAM_HINT") != nullptr;
+  face_plan(b);
   b.sh = std::make_shared<StreamHolder>();
   HIPCHK(hipStreamCreateWithFlags(&b.sh->s, hipStreamNonBlocking));
   b.stream = b.sh->s;
@@ -1261,7 +1305,7 @@ int fsil_set_boundary_conditions(int h) {
     HIPCHK(hipMemcpyAsync(b->nb_u[face].p, uu.data(), 3 * np * sizeof(double), hipMemcpyHostToDevice, b->stream));
     HIPCHK(hipStreamSynchronize(b->stream));
   }
-  if (launch_faces(*b)) return 1;
+  if (launch_faces(*b, false)) return 1;
   HIPCHK(hipStreamSynchronize(b->stream));
   return 0;
 }
@@ -1390,10 +1434,10 @@ int fsil_collide_stream_bc(int h) {
   if (!b) return 1;
   if (b->precision == 0) {
     if (collide_stream(*b)) return 1;
-    if (launch_faces(*b)) return 1;
+    if (launch_faces(*b, true)) return 1;
   } else {
     if (collide_stream32(*b)) return 1;
-    if (launch_faces(*b)) return 1;
+    if (launch_faces(*b, true)) return 1;
   }
   b->ibm.active = false;
   return 0;
@@ -2223,7 +2267,7 @@ int fsil_fsi_step(int h, double time, int numsubstep, int *iters, double *dmax) 
     if (rc) return 1;
     HIPCHK(hipStreamWaitEvent(b->stream, b->ibm.rep->ev, 0));
     if (collide_any(*b, kRegionHull, hole)) return 1;
-    if (launch_faces(*b)) return 1;
+    if (launch_faces(*b, true)) return 1;
     b->ibm.active = false;
     return fsil_ibm_report(h, iters, dmax);
   }
@@ -2560,7 +2604,7 @@ int tree_step(Block &b) {
   update_vf(b);
   if (extract_layer(b, 1)) return 1;
   if (collide_stream(b)) return 1;
-  if (launch_faces(b)) return 1;
+  if (launch_faces(b, true)) return 1;
   b.ibm.active = false;
   if (extract_layer(b, 2)) return 1;
   for (auto &pp : b.sons) {

@@ -35,6 +35,7 @@ struct Collide32Args {
   int nt;    // nontemporal population loads and stores (selects the kernel instantiation)
   int zrow;  // workgroups are whole z-rows: 1 shift_rows_z, 2 shift_rows_z_waves (rows of
              // whole waves)
+  ZFaces zf;    // z faces applied in the launch (zrow only)
   int region;   // CollideRegion
   int hole[4];  // kRegionBulk / kRegionHull: x0, x1, y0, y1
   // auxiliary planes of boundary codes 102 (den/u of the first interior
@@ -252,17 +253,24 @@ __device__ __forceinline__ void collide_push32_cell(const Collide32Args &a, int 
       if (on && c == (hi ? nd - 1 : 0)) {
         const int p = face_plane_index(face, x, y, z, a.yd, a.zd);
         const int np = axis == 0 ? a.yd * a.zd : (axis == 1 ? a.xd * a.zd : a.xd * a.yd);
-        for (int q = 0; q < Q; ++q) a.hw[face][(long long)q * np + p] = (double)post[q] + wt(q);
+        save_face(a.hw[face], face, np, p, post);
       }
     }
   }
+  float hw[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+  if (a.zf.halfway()) face_bound(hw, post, z);
   if (a.zrow) {
     if (a.zrow == 2) shift_rows_z_waves(post, zx);
     else shift_rows_z(post, zx);
     if (!on) return;
   }
   const unsigned st[6] = {sxp, sxm, syp, sym, a.zrow ? 0u : szp, a.zrow ? 0u : szm};
-  store_cell(post, a.gout, plane, n, st, NT);
+  if (a.zf.walls()) {
+    store_cell_faces(post, hw, a.gout, plane, n, st, NT, a.zf, x, y, z, a.xd, a.yd, a.zd);
+  } else {
+    if (a.zf.any()) mirror_faces(post, a.zf, x, y, z, a.xd, a.yd, a.zd);
+    store_cell(post, a.gout, plane, n, st, NT);
+  }
 }
 
 // The z-row exchange has workgroup barriers: a workgroup of whole z-rows is

@@ -153,6 +153,7 @@ struct CollideArgs {
   int region;                     // CollideRegion
   int hole[4];                    // kRegionBulk / kRegionHull: x0, x1, y0, y1
   int zrow;                       // workgroups are whole z-rows (shift_rows_z)
+  ZFaces zf;                      // z faces applied in the launch (zrow only)
 };
 
 // velocity of one cell as the collision reads it: the moments of the stored
@@ -202,6 +203,17 @@ __device__ __forceinline__ int face_plane_index(int face, int x, int y, int z, i
   if (axis == 0) return y * zd + z;
   if (axis == 1) return x * zd + z;
   return x * yd + y;
+}
+
+// The post-collision populations of a boundary node that the halfway walls of
+// `face` send back (moving into the face), into its plane buffer [q][np]
+template <typename T>
+__device__ __forceinline__ void save_face(double *hw, int face, int np, int p, const T (&post)[Q]) {
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int e = (face >> 1) == 0 ? ex(q) : ((face >> 1) == 1 ? ey(q) : ez(q));
+    if (e == ((face & 1) ? 1 : -1)) hw[(long long)q * np + p] = sizeof(T) == 8 ? (double)post[q] : (double)post[q] + wt(q);
+  }
 }
 
 // One cell: load its 19 pre-collision populations, collide, push the 19
@@ -405,7 +417,7 @@ __device__ __forceinline__ void collide_push_cell(const CollideArgs &a, int x, i
       if (on && c == (hi ? nd - 1 : 0)) {
         const int p = face_plane_index(face, x, y, z, a.yd, a.zd);
         const int np = axis == 0 ? a.yd * a.zd : (axis == 1 ? a.xd * a.zd : a.xd * a.yd);
-        for (int q = 0; q < Q; ++q) a.hw[face][(long long)q * np + p] = post[q];
+        save_face(a.hw[face], face, np, p, post);
       }
     }
   }
@@ -419,12 +431,20 @@ __device__ __forceinline__ void collide_push_cell(const CollideArgs &a, int x, i
   const unsigned sym = y == 0 ? (unsigned)(a.yd - 1) * zd : 0u - zd;
   const unsigned szp = z + 1 == a.zd ? 0u - (unsigned)(a.zd - 1) : 1u;
   const unsigned szm = z == 0 ? (unsigned)(a.zd - 1) : 0u - 1u;
+  double hw[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  if constexpr (AUX)
+    if (a.zf.halfway()) face_bound(hw, post, z);
   if (a.zrow) {
     shift_rows_z(post, zx);
     if (!on) return;
   }
   const unsigned st[6] = {sxp, sxm, syp, sym, a.zrow ? 0u : szp, a.zrow ? 0u : szm};
-  store_cell(post, a.fout, plane, n, st, NT);
+  if (a.zf.walls()) {
+    store_cell_faces(post, hw, a.fout, plane, n, st, NT, a.zf, x, y, z, a.xd, a.yd, a.zd);
+  } else {
+    if (a.zf.any()) mirror_faces(post, a.zf, x, y, z, a.xd, a.yd, a.zd);
+    store_cell(post, a.fout, plane, n, st, NT);
+  }
 }
 
 // Bound: HBM (304 bytes per cell).  With the z-moving values exchanged so
@@ -729,6 +749,47 @@ template <int AXIS, bool F32>
 __global__ __launch_bounds__(256) void k_face_pair(FaceArgs lo, FaceArgs hi, int nblk) {
   if ((int)blockIdx.x < nblk) face_node<2 * AXIS, F32>(lo, blockIdx.x * blockDim.x + threadIdx.x);
   else face_node<2 * AXIS + 1, F32>(hi, ((int)blockIdx.x - nblk) * blockDim.x + threadIdx.x);
+}
+
+// The faces of a block whose z faces the collide launch applies (ZFaces) or
+// has none of: the nodes of the active x and y faces in one launch, one thread
+// per node applying its x, y and z faces in that order.  The y and z codes set
+// a node from its own populations alone (or from its halfway plane), so only
+// the x faces read other nodes: the next two inward, which another thread may
+// be completing.  What it overwrites there are populations coming out of a y
+// or z face that the reading node is on as well, and whose own y or z face
+// overwrites them again: the value read does not matter.
+struct RimArgs {
+  FaceArgs f[6];
+  int active;  // bit k: face k
+};
+template <bool F32>
+__global__ __launch_bounds__(256) void k_rim(RimArgs a) {
+  const int xd = a.f[0].xd, yd = a.f[0].yd, zd = a.f[0].zd;
+  const int xlo = a.active & 1, xhi = (a.active >> 1) & 1, ylo = (a.active >> 2) & 1, yhi = (a.active >> 3) & 1;
+  int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int nx = (xlo + xhi) * yd * zd, w = xd - xlo - xhi;
+  int x, y, z;
+  if (t < nx) {
+    const int p = t / (yd * zd), r = t - p * yd * zd;
+    x = p == 0 && xlo ? 0 : xd - 1;
+    y = r / zd;
+    z = r - y * zd;
+  } else {
+    t -= nx;
+    if (t >= (ylo + yhi) * w * zd) return;
+    const int p = t / (w * zd), r = t - p * w * zd;
+    y = p == 0 && ylo ? 0 : yd - 1;
+    x = r / zd;
+    z = r - x * zd;
+    x += xlo;
+  }
+  if (x == 0 && xlo) face_node<0, F32>(a.f[0], y * zd + z);
+  if (x == xd - 1 && xhi) face_node<1, F32>(a.f[1], y * zd + z);
+  if (y == 0 && ylo) face_node<2, F32>(a.f[2], x * zd + z);
+  if (y == yd - 1 && yhi) face_node<3, F32>(a.f[3], x * zd + z);
+  if (z == 0 && (a.active & 16)) face_node<4, F32>(a.f[4], x * yd + y);
+  if (z == zd - 1 && (a.active & 32)) face_node<5, F32>(a.f[5], x * yd + y);
 }
 
 }  // namespace fsil
