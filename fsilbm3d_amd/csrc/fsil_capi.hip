@@ -1068,10 +1068,12 @@ int fsil_block_create(int id, const int *dims, const double *geom, const int *bc
     // The coupling's small launches and the beam's workgroups wait for CU
     // slots while the bulk's workgroups fill every CU.  The bulk asks for
     // enough LDS that at most R of its workgroups share a CU
-    // (FSIL_BULK_RESIDENCY=R, default 2; 0: no limit).  Measured, ms for the
-    // same run at R = 2, 3, 4, 5: FP64 31.0, 31.2, 32.4, 33.7; sixty steps in
-    // FP32-deviation form 37.1, 37.2, 39.2, 40.0.
-    int R = 2;
+    // (FSIL_BULK_RESIDENCY=R, default 3; 0: no limit): fewer leave the bulk
+    // short of waves, more starve the coupling.  Measured, ms for the same run
+    // at R = 2 and 3: FP64 31.0 and 30.6, sixty steps in FP32-deviation form
+    // 38.0 and 35.0 (at 4 and 5, with the faces still launches of their own:
+    // 32.4 and 33.7, 39.2 and 40.0).
+    int R = 3;
     if (const char *r = getenv("FSIL_BULK_RESIDENCY")) R = atoi(r);
     int dev = 0, per_cu = 0;
     HIPCHK(hipGetDevice(&dev));
