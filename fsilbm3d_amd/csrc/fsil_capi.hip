@@ -141,11 +141,14 @@ struct Ibm {
   // device: stencils and band (built each call, see fsil_ibm_kernels.h)
   int cap = 0;                               // 64*M, stride of the band arrays
   DevBuf<float> dEw;                         // 12*M
-  DevBuf<float4> went;                       // per band entry (CSR order): rx, ry, rz
+  DevBuf<float4> went;                       // per band entry (CSR order): rx, ry, rz, its marker
+  bool one_launch = false;                   // the forcing rounds in one launch (k_rounds), then:
+  DevBuf<int4> ecell;                        // per stencil entry: its cell, the cell's range, its rank in it
+  DevBuf<double> xch;                        // the markers' forces and residual terms, two copies
   DevBuf<unsigned> keys;                      // cell of each stencil entry
   DevBuf<int> tmp;                            // entries in arrival order per band cell
   DevBuf<int> blkbox;                         // per claim workgroup: its part of the band's box
-  DevBuf<int> flags, scan, dentry, dbidx, dptr, ctl, cellmap;
+  DevBuf<int> flags, scan, dbidx, dptr, ctl, cellmap;
   DevBuf<long long> dcell;
   DevBuf<double> band_u, band_F, dstate;
   std::unique_ptr<PinnedReport> rep = std::make_unique<PinnedReport>();
@@ -1494,6 +1497,19 @@ int fsil_time_steps(int h, int nsteps, double t0, double dt, double *total_ms) {
 
 // ---------------------------------------------------------------------------
 // immersed boundary
+// whether the forcing rounds run in one launch: its workgroups have to be
+// resident together
+static int ibm_rounds_rule(Ibm &I) {
+  int dev = 0, cus = 0;
+  HIPCHK(hipGetDevice(&dev));
+  HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  constexpr int per = kRoundsThreads / 64;
+  I.one_launch = I.M > 0 && I.M <= std::min(kRoundsMarkers, cus / kRoundsShare * per);
+  if (const char *e = getenv("FSIL_ROUNDS"))
+    if (atoi(e) == 0) I.one_launch = false;
+  return 0;
+}
+
 int fsil_ibm_define_bodies(int h, int nbodies, const int *nmarkers, const int *nnodes,
                            const int *nelems, const int *marker_elem, const int *elem_nodes) {
   Block *b = get_block(h);
@@ -1576,12 +1592,16 @@ int fsil_ibm_define_bodies(int h, int nbodies, const int *nmarkers, const int *n
   HIPCHK(I.blkbox.ensure(6 * (size_t)((I.cap + kClaimThreads - 1) / kClaimThreads)));
   HIPCHK(I.flags.ensure(I.cap));
   HIPCHK(I.scan.ensure((size_t)I.cap + kScanRun));  // k_band_scan reads whole runs of kScanRun
-  HIPCHK(I.dentry.ensure(I.cap));
   HIPCHK(I.went.ensure(I.cap));
   HIPCHK(I.dbidx.ensure(I.cap));
   HIPCHK(I.dptr.ensure((size_t)I.cap + 1));
   HIPCHK(I.dcell.ensure(I.cap));
   HIPCHK(I.band_u.ensure(3 * (size_t)I.cap));
+  if (ibm_rounds_rule(I)) return 1;
+  if (I.one_launch) {
+    HIPCHK(I.ecell.ensure(I.cap));
+    HIPCHK(I.xch.ensure(8 * (size_t)I.M));
+  }
   HIPCHK(I.band_F.ensure(3 * (size_t)I.cap));
   HIPCHK(I.dstate.ensure(4));
   HIPCHK(I.tolpart.ensure(std::max(1, I.M)));  // per-marker |dV|_1
@@ -1663,6 +1683,8 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
   }
   // the guess needs the previous call's force (Eprev) and the skip within the loop's cap
   const int warm = (net && !done0 && I.have_prev && I.skip < I.ntol) ? 1 : 0;
+  // the plain loop in one launch where its workgroups fit (k_rounds)
+  const bool one_launch = I.one_launch && !done0 && !net && !I.record;
   hipLaunchKernelGGL(k_ibm_reset, dim3(std::min(1024, (E + 255) / 256)), dim3(256), 0, s, I.ctl.p, I.dcell.p,
                      I.cellmap.p, I.dstate.p, done0, warm, I.skip, E, I.scan.p, I.dptr.p, I.Eforce.p, 3 * M);
   HIPCHK(hipGetLastError());
@@ -1700,7 +1722,7 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
   hipLaunchKernelGGL(k_ibm_fill, dim3((E + 255) / 256), dim3(256), 0, s, E, I.dbidx.p, I.flags.p, I.dptr.p,
                      I.tmp.p);
   hipLaunchKernelGGL(k_ibm_rank, dim3((E + 255) / 256), dim3(256), 0, s, E, I.ctl.p, I.dbidx.p, I.dptr.p, I.tmp.p,
-                     I.dentry.p, I.dEw.p, I.went.p);
+                     I.dEw.p, I.went.p, one_launch ? I.ecell.p : nullptr);
   HIPCHK(hipGetLastError());
   const double invh3p = 0.5 * dt * ((1.0 / b->dh) * (1.0 / b->dh) * (1.0 / b->dh)) / I.denIn;
   double dsum = 0.0;
@@ -1717,7 +1739,7 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
     hipLaunchKernelGGL(k_ws_apply, dim3((3 * M + 255) / 256), dim3(256), 0, s, M, I.wsP.p, I.Ea.p, I.Eprev.p, I.Uref,
                        invh3p, I.Eforce.p, I.fT.p);
     hipLaunchKernelGGL(k_correct, dim3(cell_blocks), dim3(256), 0, s, I.ctl.p, -1, MdfTest{}, I.cap, I.dptr.p,
-                       I.dentry.p, I.went.p, I.fT.p, I.band_u.p, cell_blocks, I.pass_cap);
+                       I.went.p, I.fT.p, I.band_u.p, cell_blocks, I.pass_cap);
     HIPCHK(hipGetLastError());
   }
   // MDF loop (Solidbody.f90:893-906): the rounds are queued (with the warm
@@ -1730,12 +1752,21 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
   MdfTest mt{};
   mt.tl = I.tolpart.p; mt.dstate = I.dstate.p; mt.M = M; mt.ntol = I.ntol;
   mt.dsum = dsum; mt.Uref = I.Uref; mt.dtol = I.dtol; mt.skip = I.skip;
-  for (int it = 0; it < rounds; ++it) {
+  if (one_launch) {
+    RoundsArgs ra{};
+    ra.M = M; ra.cap = I.cap; ra.ctl = I.ctl.p;
+    ra.Ew = I.dEw.p; ra.went = I.went.p; ra.ecell = I.ecell.p; ra.Evel = I.Evel.p; ra.Ea = I.Ea.p;
+    ra.invh3 = invh3p; ra.Eforce = I.Eforce.p; ra.band_u = I.band_u.p; ra.xch = I.xch.p; ra.mt = mt;
+    constexpr int per = kRoundsThreads / 64;
+    hipLaunchKernelGGL(k_rounds, dim3((M + per - 1) / per), dim3(kRoundsThreads), 0, s, ra);
+    HIPCHK(hipGetLastError());
+  }
+  for (int it = 0; it < rounds && !one_launch; ++it) {
     hipLaunchKernelGGL(k_interp, dim3((M + 3) / 4), dim3(256), 0, s, M, it, I.dbidx.p, I.dEw.p, I.band_u.p, I.cap,
                        I.ctl.p, I.Evel.p, I.Ea.p, invh3p, I.Eforce.p, I.fT.p, I.tolpart.p, snap, I.Esnap.p);
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(k_correct, dim3(cell_blocks + 1), dim3(256), 0, s, I.ctl.p, it, mt, I.cap, I.dptr.p,
-                       I.dentry.p, I.went.p, I.fT.p, I.band_u.p, cell_blocks, I.pass_cap);
+                       I.went.p, I.fT.p, I.band_u.p, cell_blocks, I.pass_cap);
     HIPCHK(hipGetLastError());
     if (warm && it == 0) {
       // restart from the zero guess when the first round asked for it
@@ -1760,7 +1791,7 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
   // spreading (Solidbody.f90:920-979), beam loads and the report in one launch
   IbmFinishArgs fa{};
   fa.ctl = I.ctl.p; fa.dstate = I.dstate.p; fa.rep = I.rep->d;
-  fa.cap = I.cap; fa.ptr = I.dptr.p; fa.entry = I.dentry.p; fa.went = I.went.p; fa.Eforce = I.Eforce.p;
+  fa.cap = I.cap; fa.ptr = I.dptr.p; fa.went = I.went.p; fa.Eforce = I.Eforce.p;
   fa.invh3 = (1.0 / b->dh) * (1.0 / b->dh) * (1.0 / b->dh);
   fa.VF1 = b->VF[0]; fa.VF2 = b->VF[1]; fa.VF3 = b->VF[2];
   fa.band_F = I.band_F.p;
@@ -1869,6 +1900,7 @@ int ibm_check_report(Block &b) {
   if (err != 0x7fffffff) {
     I.active = false;
     if (err == 3) return fail("Nan found in PenaltyForce");
+    if (err == 2) return fail("forcing rounds: a workgroup did not start in time");
     if (err == 4) return fail("immersed-boundary band: a stencil cell without a band number");
     const int m = err / 4 - 1, why = err % 4;
     int body = 0;

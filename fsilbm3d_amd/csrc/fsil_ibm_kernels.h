@@ -42,6 +42,7 @@ enum IbmCtl {
   kRan = 14,       // the last forcing round whose interpolation ran (-1: none)
   kGuess = 15,     // 1: the learned guess was applied in this call (kept on fallback)
   kSkip = 16,      // forcing rounds the applied guess stands for (0 without a guess)
+  kArrived = 17,   // workgroups of k_rounds that reached its barriers so far
   kCtlWords = 20
 };
 
@@ -97,6 +98,7 @@ __global__ __launch_bounds__(256) void k_ibm_reset(int *__restrict__ ctl, const 
     band_ptr[0] = 0;
     ctl[kNew] = 0;
     ctl[kRan] = -1;
+    ctl[kArrived] = 0;
     ctl[kErr] = 0x7fffffff;
     ctl[kDone] = done0;
     // a learned guess stands for the first `skip` forcing rounds: the loop
@@ -285,12 +287,13 @@ __global__ __launch_bounds__(256) void k_ibm_fill(int E, const int *__restrict__
 
 // every entry at its rank in its cell's range (the number of the cell's
 // entries below it, its range read sixteen entries at a time), so each cell
-// lists its entries in ascending e, its weights (rx, ry, rz) beside it in
-// went; the band size is published
+// lists its entries in ascending e: went holds an entry's weights (rx, ry,
+// rz) and its marker, ecell (where k_rounds runs) an entry's cell, the cell's
+// range and the entry's rank in it; the band size is published
 __global__ __launch_bounds__(256) void k_ibm_rank(int E, int *__restrict__ ctl, const int *__restrict__ bidx,
                                                   const int *__restrict__ band_ptr, const int *__restrict__ tmp,
-                                                  int *__restrict__ entry, const float *__restrict__ Ew,
-                                                  float4 *__restrict__ went) {
+                                                  const float *__restrict__ Ew, float4 *__restrict__ went,
+                                                  int4 *__restrict__ ecell) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e == 0) ctl[kNband] = ctl[kNew];
   if (e >= E) return;
@@ -308,9 +311,9 @@ __global__ __launch_bounds__(256) void k_ibm_rank(int E, int *__restrict__ ctl, 
 #pragma unroll
     for (int j = 0; j < 16; ++j) r += v[j] < e ? 1 : 0;
   }
-  entry[p0 + r] = e;
-  // the entry's three stencil weights beside it, in the cells' order
-  went[p0 + r] = make_float4(wx, wy, wz, 0.0f);
+  // the entry's three stencil weights and its marker, in the cells' order
+  went[p0 + r] = make_float4(wx, wy, wz, __int_as_float(m));
+  if (ecell) ecell[e] = make_int4(b, p0, n, r);
 }
 
 // band macros: den/u of every band cell from the stored state, same
@@ -563,8 +566,8 @@ __global__ __launch_bounds__(256) void k_interp(int M, int round, const int *__r
 // The per-cell sums over a band cell's entries (the velocity correction and
 // the spreading), by workgroups of 256 threads taking kCellsPerPass
 // consecutive cells at a time: the cells' entries are one contiguous range of
-// the CSR arrays, so each thread forms one entry's term from coalesced reads
-// (entry, weights) and one gather (the marker's value) into LDS, and then one
+// the CSR arrays, so each thread forms one entry's term from one coalesced
+// read (weights and marker) and one gather (the marker's value) into LDS, and then one
 // thread per cell adds its terms in entry order, as the sequential loop does.
 // A pass whose range exceeds the LDS area (pass_cap <= kPassEntries entries)
 // falls back to one thread per cell reading its entries itself.  SPREAD: term = -(((v h^-3 rx)
@@ -574,9 +577,9 @@ constexpr int kCellsPerPass = 32;
 constexpr int kPassEntries = 1024;  // 24 KiB of LDS: fits beside the bulk collide of a split step
 template <bool SPREAD>
 __device__ inline void band_cells_reduce(int blk, int nb, int nblk, int cap, const int *__restrict__ ptr,
-                                         const int *__restrict__ entry, const float4 *__restrict__ went,
-                                         const double *__restrict__ val, double invh3, double *__restrict__ out,
-                                         double VF1, double VF2, double VF3, int pass_cap) {
+                                         const float4 *__restrict__ went, const double *__restrict__ val,
+                                         double invh3, double *__restrict__ out, double VF1, double VF2,
+                                         double VF3, int pass_cap) {
   __shared__ int sptr[kCellsPerPass + 1];
   __shared__ double term[3][kPassEntries];
   const int t = threadIdx.x;
@@ -594,8 +597,8 @@ __device__ inline void band_cells_reduce(int blk, int nb, int nblk, int cap, con
     const bool fits = ne <= pass_cap;
     if (fits) {
       for (int k = t; k < ne; k += blockDim.x) {
-        const int m = entry[e0 + k] >> 6;
         const float4 w = went[e0 + k];
+        const int m = __float_as_int(w.w);
         const double rx = (double)w.x, ry = (double)w.y, rz = (double)w.z;
         double v1 = val[3LL * m], v2 = val[3LL * m + 1], v3 = val[3LL * m + 2];
         if (SPREAD) {
@@ -618,8 +621,8 @@ __device__ inline void band_cells_reduce(int blk, int nb, int nblk, int cap, con
         if (fits) {
           x1 = term[0][k]; x2 = term[1][k]; x3 = term[2][k];
         } else {
-          const int m = entry[e0 + k] >> 6;
           const float4 w = went[e0 + k];
+          const int m = __float_as_int(w.w);
           const double rx = (double)w.x, ry = (double)w.y, rz = (double)w.z;
           double v1 = val[3LL * m], v2 = val[3LL * m + 1], v3 = val[3LL * m + 2];
           if (SPREAD) {
@@ -667,7 +670,6 @@ struct MdfTest {
 // warm-start guess): runs unless the loop is done, no stop test.
 __global__ __launch_bounds__(256) void k_correct(int *__restrict__ ctl, int round, MdfTest mt, int cap,
                                                  const int *__restrict__ ptr,
-                                                 const int *__restrict__ entry,
                                                  const float4 *__restrict__ went,
                                                  const double *__restrict__ fT,
                                                  double *__restrict__ band_u, int cell_blocks, int pass_cap) {
@@ -684,8 +686,196 @@ __global__ __launch_bounds__(256) void k_correct(int *__restrict__ ctl, int roun
     return;
   }
   if (round >= 0 ? ctl[kRan] != round : ctl[kDone] != 0) return;  // uniform over the grid
-  band_cells_reduce<false>(blockIdx.x, ctl[kNband], cell_blocks, cap, ptr, entry, went, fT, 1.0, band_u, 0.0, 0.0,
-                           0.0, pass_cap);
+  band_cells_reduce<false>(blockIdx.x, ctl[kNband], cell_blocks, cap, ptr, went, fT, 1.0, band_u, 0.0, 0.0, 0.0,
+                           pass_cap);
+}
+
+// All forcing rounds of a call in one launch, one wave per marker, for marker
+// counts whose workgroups are all resident at once (kRoundsShare).
+// Lane s of a wave holds the velocity of the band cell of the marker's entry
+// s and the cell's entries (weights and markers, the first kRoundEntries of
+// them in registers) for the whole loop, so a cell's correction is formed by
+// the wave of every marker whose stencil holds it and the only values that
+// cross workgroups are the markers' forces and residual terms: a round is one
+// exchange behind one barrier instead of two launches.  Every sum is formed in
+// the order of k_interp, band_cells_reduce and mdf_tl_sum, and every workgroup
+// makes the same stop test; workgroup 0 records it.
+// The exchange goes through device-scope atomics (the workgroups run on
+// several XCDs) in two copies taken in turn: a workgroup writes round r+2's
+// values only after all have passed barrier r+1, that is, have read round r's.
+// A wait is bounded by kRoundsWait; the call then fails.
+// Bound by the exchange: about 4.5 us per round (store, count, poll and load
+// across the XCDs 3, ordered sums 1) where two launches took 9.7.  Ten rounds:
+// 144 markers 97 -> 49 us; a whole coupling call of markers 0.9 x 0.7 cells
+// apart 198 -> 160 us (256 markers), 206 -> 181 (512); with 512 markers in a
+// few cells 1676 -> 863.
+struct RoundsArgs {
+  int M, cap;
+  int *ctl;
+  const float *Ew;
+  const float4 *went;
+  const int4 *ecell;
+  const double *Evel, *Ea;
+  double invh3;
+  double *Eforce, *band_u;
+  double *xch;  // [2][4][M]: h^-3 F dt / (2 rho) per axis, |dV|_1
+  MdfTest mt;
+};
+
+constexpr int kRoundsThreads = 256;   // four markers per workgroup
+constexpr int kRoundEntries = 16;     // entries of a cell held in registers (a plane of markers a cell apart: all)
+// Every workgroup of the launch waits for every other, so all have to be
+// resident together: at most half as many as the CUs, of which each holds two
+// (173 VGPRs), so the launches of a process's four hardware queues fit at once,
+// and other kernels beside them end by themselves.  The repeated corrections
+// grow with the markers per workgroup's share of a CU; at the line (512
+// markers on 256 CUs) the form is still the faster one by 6-12%.
+constexpr int kRoundsShare = 2;
+constexpr int kRoundsMarkers = 512;   // (the exchanged values are kept in LDS)
+constexpr long long kRoundsWait = 1000000000LL;  // ticks of the 100 MHz clock: 10 s
+
+__device__ __forceinline__ double xload(const double *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void xstore(double *p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(kRoundsThreads, 2) void k_rounds(RoundsArgs a) {
+  constexpr int NW = kRoundsThreads / 64, B = kRoundEntries;
+  __shared__ double t[NW][3][64];
+  __shared__ double fx[4][kRoundsMarkers];
+  __shared__ double part[4];
+  __shared__ int late;
+  const int w = threadIdx.x >> 6, s = threadIdx.x & 63;
+  const int m = blockIdx.x * NW + w;
+  const int M = a.M, cap = a.cap;
+  const bool on = m < M;
+  const int me = on ? m : M - 1;  // (a spare wave follows the last marker and stores nothing)
+  if (threadIdx.x == 0) late = 0;
+  const int4 ec = a.ecell[64LL * me + s];
+  const float *W = a.Ew + 12LL * me;
+  const double rx = (double)W[s >> 4], ry = (double)W[4 + ((s >> 2) & 3)], rz = (double)W[8 + (s & 3)];
+  const MdfWords wd0 = mdf_words(a.ctl, a.mt.dstate);
+  // lane c < 3: component c of the marker
+  const int c = min(s, 2);
+  const double ev = a.Evel[3LL * me + c], am = a.Ea[me];
+  double ef = a.Eforce[3LL * me + c];
+  double u1 = a.band_u[ec.x], u2 = a.band_u[cap + ec.x], u3 = a.band_u[2LL * cap + ec.x];
+  const int n = ec.z;
+  const float4 *we = a.went + ec.y;
+  float4 q[B];
+#pragma unroll
+  for (int j = 0; j < B; ++j) {
+    q[j] = we[max(min(j, n - 1), 0)];
+    q[j].w = __int_as_float((int)min((unsigned)__float_as_int(q[j].w), (unsigned)(M - 1)));
+  }
+  const int nmax = [&] {
+    int v = n;
+    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
+    return __builtin_amdgcn_readfirstlane(v);
+  }();
+  MdfWords wd = wd0;
+  for (int r = 0;; ++r) {
+    t[w][0][s] = ((u1 * rx) * ry) * rz;
+    t[w][1][s] = ((u2 * rx) * ry) * rz;
+    t[w][2][s] = ((u3 * rx) * ry) * rz;
+    wave_sync();
+    double *xo = a.xch + (long long)(r & 1) * 4 * M;
+    {
+      double v = 0.0;
+#pragma unroll 16
+      for (int k = 0; k < 64; ++k) v = v + t[w][c][k];
+      const double d = ev - v, F = d * am;
+      ef = ef + F;
+      const double d0 = __shfl(d, 0, 64), d1 = __shfl(d, 1, 64), d2 = __shfl(d, 2, 64);
+      if (on && s < 4) xstore(&xo[(long long)s * M + m], s < 3 ? F * a.invh3 : (fabs(d0) + fabs(d1)) + fabs(d2));
+    }
+    // every store of this workgroup has reached memory, then it is counted
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      __hip_atomic_fetch_add(&a.ctl[kArrived], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int want = (int)gridDim.x * (r + 1);
+      const long long t0 = (long long)wall_clock64();
+      while (__hip_atomic_load(&a.ctl[kArrived], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want) {
+        if ((long long)wall_clock64() - t0 > kRoundsWait) {
+          late = 1;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+    }
+    __syncthreads();
+    if (late) {
+      if (threadIdx.x == 0) atomicMin(&a.ctl[kErr], 2);
+      return;
+    }
+    for (int i = threadIdx.x; i < M; i += kRoundsThreads) {
+      double v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = xload(&xo[(long long)k * M + i]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) fx[k][i] = v[k];
+    }
+    __syncthreads();
+    // the residual, in mdf_tl_sum's order (256 strided sums, wave trees, the four in order)
+    if (threadIdx.x < 256) {
+      double p = 0.0;
+      for (int i = threadIdx.x; i < M; i += 256) p = p + fx[3][i];
+      p = wave_sum(p);
+      if (s == 0) part[w] = p;
+    }
+    // the correction of this lane's cell, its entries in order
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+      if (j % 4 == 0 && j >= nmax) break;
+      // (the weights stay FP32 in their registers: widened copies and LDS
+      // addresses kept across the rounds would double them)
+      float4 g = q[j];
+      asm volatile("" : "+v"(g.x), "+v"(g.y), "+v"(g.z), "+v"(g.w));
+      const int k = __float_as_int(g.w);
+      const double qx = (double)g.x, qy = (double)g.y, qz = (double)g.z;
+      const double x1 = ((fx[0][k] * qx) * qy) * qz, x2 = ((fx[1][k] * qx) * qy) * qz,
+                   x3 = ((fx[2][k] * qx) * qy) * qz;
+      u1 = j < n ? u1 - x1 : u1;
+      u2 = j < n ? u2 - x2 : u2;
+      u3 = j < n ? u3 - x3 : u3;
+    }
+    for (int j0 = B; j0 < n; j0 += 8) {
+      float4 g[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) g[j] = we[min(j0 + j, n - 1)];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int k = (int)min((unsigned)__float_as_int(g[j].w), (unsigned)(M - 1));
+        const double qx = (double)g[j].x, qy = (double)g[j].y, qz = (double)g[j].z;
+        const double x1 = ((fx[0][k] * qx) * qy) * qz, x2 = ((fx[1][k] * qx) * qy) * qz,
+                     x3 = ((fx[2][k] * qx) * qy) * qz;
+        u1 = j0 + j < n ? u1 - x1 : u1;
+        u2 = j0 + j < n ? u2 - x2 : u2;
+        u3 = j0 + j < n ? u3 - x3 : u3;
+      }
+    }
+    __syncthreads();
+    double tol = 0.0;
+    for (int k = 0; k < 4; ++k) tol = tol + part[k];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      wd.iters = r;
+      mdf_decide(a.ctl, a.mt.dstate, tol, a.mt.dsum, a.mt.Uref, a.mt.ntol, a.mt.dtol, a.mt.skip, wd);
+    }
+    // (mdf_decide's condition without a learned guess, after r + 1 iterations)
+    if (!isfinite(tol) || !(r + 1 < a.mt.ntol && tol / (a.mt.dsum * a.mt.Uref) > a.mt.dtol)) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl[kRan] = r;
+      break;
+    }
+  }
+  if (on && s < 3) a.Eforce[3LL * m + s] = ef;
+  if (on && ec.w == 0) {  // the cell's first entry
+    a.band_u[ec.x] = u1;
+    a.band_u[cap + ec.x] = u2;
+    a.band_u[2LL * cap + ec.x] = u3;
+  }
 }
 
 // Inclusive scan of the per-cell entry counts of the band's cells (ctl[kNew],
@@ -804,7 +994,7 @@ struct IbmFinishArgs {
   const double *dstate;
   IbmReport *rep;
   int cap;
-  const int *ptr, *entry;
+  const int *ptr;
   const float4 *went;
   const double *Eforce;
   double invh3, VF1, VF2, VF3;
@@ -851,8 +1041,8 @@ __global__ __launch_bounds__(256) void k_ibm_finish(IbmFinishArgs a) {
   const int blk = (int)blockIdx.x - a.dof_blocks;
   if (blk == 0 && threadIdx.x < kCtlWords) a.rep->ctl[threadIdx.x] = a.ctl[threadIdx.x];
   if (blk == 0 && threadIdx.x == 0) a.rep->dmax = a.dstate[0];
-  band_cells_reduce<true>(blk, a.ctl[kNband], a.band_blocks, a.cap, a.ptr, a.entry, a.went, a.Eforce, a.invh3,
-                          a.band_F, a.VF1, a.VF2, a.VF3, a.pass_cap);
+  band_cells_reduce<true>(blk, a.ctl[kNband], a.band_blocks, a.cap, a.ptr, a.went, a.Eforce, a.invh3, a.band_F,
+                          a.VF1, a.VF2, a.VF3, a.pass_cap);
 }
 
 // ---------------------------------------------------------------------------
