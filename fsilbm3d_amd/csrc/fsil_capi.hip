@@ -148,7 +148,7 @@ struct Ibm {
   DevBuf<unsigned> keys;                      // cell of each stencil entry
   DevBuf<int> tmp;                            // entries in arrival order per band cell
   DevBuf<int> blkbox;                         // per claim workgroup: its part of the band's box
-  DevBuf<int> flags, scan, dbidx, dptr, ctl, cellmap;
+  DevBuf<int> slot, dbidx, dptr, ctl, cellmap;
   DevBuf<long long> dcell;
   DevBuf<double> band_u, band_F, dstate;
   std::unique_ptr<PinnedReport> rep = std::make_unique<PinnedReport>();
@@ -1590,8 +1590,7 @@ int fsil_ibm_define_bodies(int h, int nbodies, const int *nmarkers, const int *n
   HIPCHK(I.keys.ensure(I.cap));
   HIPCHK(I.tmp.ensure(I.cap));
   HIPCHK(I.blkbox.ensure(6 * (size_t)((I.cap + kClaimThreads - 1) / kClaimThreads)));
-  HIPCHK(I.flags.ensure(I.cap));
-  HIPCHK(I.scan.ensure((size_t)I.cap + kScanRun));  // k_band_scan reads whole runs of kScanRun
+  HIPCHK(I.slot.ensure(I.cap));
   HIPCHK(I.went.ensure(I.cap));
   HIPCHK(I.dbidx.ensure(I.cap));
   HIPCHK(I.dptr.ensure((size_t)I.cap + 1));
@@ -1686,7 +1685,7 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
   // the plain loop in one launch where its workgroups fit (k_rounds)
   const bool one_launch = I.one_launch && !done0 && !net && !I.record;
   hipLaunchKernelGGL(k_ibm_reset, dim3(std::min(1024, (E + 255) / 256)), dim3(256), 0, s, I.ctl.p, I.dcell.p,
-                     I.cellmap.p, I.dstate.p, done0, warm, I.skip, E, I.scan.p, I.dptr.p, I.Eforce.p, 3 * M);
+                     I.cellmap.p, I.dstate.p, done0, warm, I.skip, I.Eforce.p, 3 * M);
   HIPCHK(hipGetLastError());
   StencilArgs sa{};
   sa.M = M;
@@ -1700,27 +1699,24 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
   sa.Ew = I.dEw.p;
   sa.keys = I.keys.p;
   sa.ctl = I.ctl.p;
-  // band: cells bid for by the stencils and claimed, per-cell counts (I.scan) and slots
-  // (I.flags), CSR pointers by an inclusive scan into dptr[1..], entries
-  // placed in arrival order (I.tmp), then at their ranks by entry number
-  sa.cellmap = I.cellmap.p;  // (the stencil kernel makes the bids)
+  // band: entries counted into their cells (slots), cells claimed with their
+  // ranges, entries placed in arrival order (I.tmp), then at their ranks
+  sa.cellmap = I.cellmap.p;
+  sa.slot = I.slot.p;
   hipLaunchKernelGGL(k_ibm_stencil, dim3((M + 3) / 4), dim3(256), 0, s, sa);
   const int nclaim = (E + kClaimThreads - 1) / kClaimThreads;
-  hipLaunchKernelGGL(k_ibm_claim, dim3(nclaim), dim3(kClaimThreads), 0, s, E, I.keys.p, I.cellmap.p, I.dcell.p,
-                     b->yd, b->zd, I.blkbox.p, I.ctl.p);
+  hipLaunchKernelGGL(k_ibm_claim, dim3(nclaim), dim3(kClaimThreads), 0, s, E, I.keys.p, I.slot.p, I.cellmap.p,
+                     I.dcell.p, I.dptr.p, b->yd, b->zd, I.blkbox.p, I.ctl.p);
   HIPCHK(hipGetLastError());
-  // calculate_interaction_force (Solidbody.f90:869-918): band velocity of the stored state with the count
+  // calculate_interaction_force (Solidbody.f90:869-918): band velocity of the stored state with the placing
   const double hv0 = 0.5 * b->VF[0] * b->dh, hv1 = 0.5 * b->VF[1] * b->dh, hv2 = 0.5 * b->VF[2] * b->dh;
   BandMacroArgs ma{};
   ma.f = b->precision == 0 ? b->fA.p : nullptr;
   ma.g = b->precision == 0 ? nullptr : b->gA.p;
   ma.N = b->N; ma.cell = I.dcell.p; ma.cap = I.cap; ma.hv0 = hv0; ma.hv1 = hv1; ma.hv2 = hv2; ma.band_u = I.band_u.p;
-  hipLaunchKernelGGL(k_ibm_count, dim3((E + 255) / 256), dim3(256), 0, s, E, I.keys.p, I.cellmap.p, I.dbidx.p,
-                     I.scan.p, I.flags.p, I.ctl.p, ma);
+  hipLaunchKernelGGL(k_ibm_fill, dim3((E + 255) / 256 + 1), dim3(256), 0, s, E, I.keys.p, I.cellmap.p, I.slot.p,
+                     I.dptr.p, I.dbidx.p, I.tmp.p, I.ctl.p, I.blkbox.p, nclaim, ma);
   HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_band_scan, dim3(1), dim3(1024), 0, s, I.ctl.p, I.scan.p, I.dptr.p, I.blkbox.p, nclaim);
-  hipLaunchKernelGGL(k_ibm_fill, dim3((E + 255) / 256), dim3(256), 0, s, E, I.dbidx.p, I.flags.p, I.dptr.p,
-                     I.tmp.p);
   hipLaunchKernelGGL(k_ibm_rank, dim3((E + 255) / 256), dim3(256), 0, s, E, I.ctl.p, I.dbidx.p, I.dptr.p, I.tmp.p,
                      I.dEw.p, I.went.p, one_launch ? I.ecell.p : nullptr);
   HIPCHK(hipGetLastError());

@@ -10,14 +10,17 @@
 //
 // The whole structure is built on the device each coupling call, with no
 // global sort: k_ibm_stencil (one wave per marker) forms the stencil and
-// every entry bids for its cell in the cell map; k_ibm_claim gives each
-// cell's winning entry a band number (from an atomic counter, so the band's
+// counts every entry into its cell in the cell map, which gives the entry a
+// slot; k_ibm_claim gives each cell's first entry a band number and the cell
+// its range of the entry list (both from one atomic counter, so the band's
 // order varies from call to call while every per-cell result does not);
-// k_ibm_count gives every entry its band cell and a slot; an inclusive scan
-// of the per-cell counts makes the CSR pointers (and the band's box);
-// k_ibm_fill places the
-// entries in arrival order and k_ibm_rank moves each to its rank by e among
-// its cell's entries.  Band arrays
+// k_ibm_fill gives every entry its band cell and places the entries in arrival
+// order, and k_ibm_rank moves each to its rank by e among its cell's entries.
+// Five launches (seven with bids for the cells, counts per band cell and a
+// scan of them), since each costs its launch and a trip to memory: kernels of
+// 144 markers 34 -> 26 us and two launch gaps, of 2304 markers beside a bulk
+// collide 76 -> 66 us.
+// Band arrays
 // have a fixed stride `cap` = 64*M (an upper bound of the band size) and the
 // band size itself lives in device memory (ctl[kNband]), so nothing is read
 // back between the kernels.
@@ -38,11 +41,12 @@ enum IbmCtl {
   kWarm = 10,      // learned warm start in use for this call
   kFallback = 11,  // 1: the warm start did not lower the residual, restart from zero; 2: restarted
   kDone0 = 12,     // the done word at the start of a loop (no iteration at all)
-  kNew = 13,       // band cells claimed so far in this call (becomes kNband)
+  kArrived = 13,   // workgroups of k_rounds that reached its barriers so far
   kRan = 14,       // the last forcing round whose interpolation ran (-1: none)
   kGuess = 15,     // 1: the learned guess was applied in this call (kept on fallback)
   kSkip = 16,      // forcing rounds the applied guess stands for (0 without a guess)
-  kArrived = 17,   // workgroups of k_rounds that reached its barriers so far
+  kNew = 18,       // band cells claimed so far in this call (becomes kNband)
+  kNewEntries = 19,  // and their entries (one 64-bit counter with kNew)
   kCtlWords = 20
 };
 
@@ -81,22 +85,20 @@ __host__ __device__ inline int trim4(int i, int nd, int *out, int bclo, int bchi
   return err;
 }
 
-// reset of the control words; clears the previous band from the cell map,
-// the per-cell entry counts (E of them) of this call and the marker forces
+// reset of the control words; clears the previous band from the cell map and
+// the marker forces
 __global__ __launch_bounds__(256) void k_ibm_reset(int *__restrict__ ctl, const long long *__restrict__ prev_cell,
                                                    int *__restrict__ cellmap, double *__restrict__ dstate,
-                                                   int done0, int warm, int skip, int E,
-                                                   int *__restrict__ count, int *__restrict__ band_ptr,
+                                                   int done0, int warm, int skip,
                                                    double *__restrict__ Eforce, int n3M) {
   const int nprev = ctl[kNband];
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nprev; i += gridDim.x * blockDim.x)
     cellmap[prev_cell[i]] = -1;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < E; i += gridDim.x * blockDim.x) count[i] = 0;
   // v_Eforce = 0 (Solidbody.f90:889)
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n3M; i += gridDim.x * blockDim.x) Eforce[i] = 0.0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    band_ptr[0] = 0;
     ctl[kNew] = 0;
+    ctl[kNewEntries] = 0;
     ctl[kRan] = -1;
     ctl[kArrived] = 0;
     ctl[kErr] = 0x7fffffff;
@@ -124,15 +126,15 @@ struct StencilArgs {
   float *__restrict__ Ew;                // 12*M
   unsigned *__restrict__ keys;           // 64*M: cell of entry e = 64*m + s
   int *__restrict__ ctl;
-  int *__restrict__ cellmap;             // the entries' bids
+  int *__restrict__ cellmap;             // entries per cell so far: -1 - their number
+  int *__restrict__ slot;                // 64*M: arrival number of the entry in its cell
 };
 
 // UpdateElmtInterp_ (Solidbody.f90:760-821), one wave per marker: every lane
 // forms the marker's anchor (from its body's first marker) and trimmed 4x3
-// indices, lanes 0..11 write the FP32 weights, lane s the cell of entry s and
-// that entry's bid in the cell map: every entry bids -(e+2) for its cell, the
-// map keeps the lowest bid, so the cell's highest entry wins (cells outside
-// the band hold -1).
+// indices, lanes 0..11 write the FP32 weights, lane s the cell of entry s, and
+// counts the entry into the cell map, where a cell of n entries so far holds
+// -1 - n (cells outside the band hold -1).
 __global__ __launch_bounds__(256) void k_ibm_stencil(StencilArgs a) {
   const int s = threadIdx.x & 63;
   const int m = blockIdx.x * 4 + ((int)threadIdx.x >> 6);
@@ -160,32 +162,36 @@ __global__ __launch_bounds__(256) void k_ibm_stencil(StencilArgs a) {
       ((unsigned)(cidx[0] - 1) * (unsigned)a.nd[1] + (unsigned)(cidx[1] - 1)) * (unsigned)a.nd[2] +
       (unsigned)(cidx[2] - 1);
   a.keys[64LL * m + s] = key;
-  // the entry's bid for its cell
-  atomicMin(&a.cellmap[key], -(64 * m + s + 2));
+  a.slot[64LL * m + s] = -1 - atomicSub(&a.cellmap[key], 1);
 }
 
 // Cell-map accesses of the band build go through device-scope atomics (the
-// workgroups that bid for, claim and look up one cell run on different XCDs).
+// workgroups that count into, claim and look up one cell run on different XCDs).
 __device__ __forceinline__ int cellmap_load(const int *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// the winning entry of each cell takes a band number and writes it into the
-// cell map.  One 1024-thread workgroup makes one atomic add on the band
-// counter (atomics on one line from many workgroups serialize), and leaves
-// its part of the band's bounding box in blkbox[6 * workgroup ..] for
-// k_band_scan.
+// The first entry of each cell takes a band number and the cell's range of the
+// entry list, whose start it leaves in ptr, and writes the number into the cell
+// map.  One 1024-thread workgroup makes one atomic add on the counter of cells
+// and entries (atomics on one line from many workgroups serialize): both are
+// handed out together, so the ranges lie in band order.  The workgroup's part
+// of the band's bounding box goes to blkbox[6 * workgroup ..] for k_ibm_fill.
 constexpr int kClaimThreads = 1024;
 __global__ __launch_bounds__(kClaimThreads) void k_ibm_claim(int E, const unsigned *__restrict__ keys,
+                                                             const int *__restrict__ slot,
                                                              int *__restrict__ cellmap,
-                                                             long long *__restrict__ band_cell, int ny, int nz,
+                                                             long long *__restrict__ band_cell,
+                                                             int *__restrict__ ptr, int ny, int nz,
                                                              int *__restrict__ blkbox, int *__restrict__ ctl) {
   constexpr int NW = kClaimThreads / 64;
-  __shared__ int wave_won[NW], wave_off[NW], blk_base, wbox[NW][6];
+  __shared__ int wave_won[NW], wave_ent[NW], wave_off[NW], wave_eoff[NW], wbox[NW][6];
+  __shared__ unsigned long long blk_base;
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   const int s = threadIdx.x & 63, w = (int)threadIdx.x >> 6;
   const unsigned cell = e < E ? keys[e] : 0u;
-  const bool won = e < E && cellmap_load(&cellmap[cell]) == -(e + 2);
+  const bool won = e < E && slot[e] == 0;
+  const int n = won ? -1 - cellmap_load(&cellmap[cell]) : 0;  // the cell's entries
   const unsigned long long mask = __ballot(won);
   int v[3];
   {
@@ -207,15 +213,28 @@ __global__ __launch_bounds__(kClaimThreads) void k_ibm_claim(int E, const unsign
       wbox[w][3 + k] = hi;
     }
   }
-  if (s == 0) wave_won[w] = __popcll(mask);
+  int upto = n;  // entries of the wave's cells up to this lane's
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int o = __shfl_up(upto, off, 64);
+    if (s >= off) upto += o;
+  }
+  if (s == 63) {
+    wave_won[w] = __popcll(mask);
+    wave_ent[w] = upto;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
-    int t = 0;
+    int t = 0, u = 0;
     for (int k = 0; k < NW; ++k) {
       wave_off[k] = t;
+      wave_eoff[k] = u;
       t += wave_won[k];
+      u += wave_ent[k];
     }
-    blk_base = t ? atomicAdd(&ctl[kNew], t) : 0;
+    blk_base = t ? atomicAdd(reinterpret_cast<unsigned long long *>(&ctl[kNew]),
+                             ((unsigned long long)u << 32) | (unsigned long long)t)
+                 : 0ULL;
   }
   if (threadIdx.x < 6) {
     const int k = threadIdx.x;
@@ -225,8 +244,9 @@ __global__ __launch_bounds__(kClaimThreads) void k_ibm_claim(int E, const unsign
   }
   __syncthreads();
   if (won) {
-    const int b = blk_base + wave_off[w] + __popcll(mask & ((1ULL << s) - 1ULL));
+    const int b = (int)(blk_base & 0xffffffffULL) + wave_off[w] + __popcll(mask & ((1ULL << s) - 1ULL));
     band_cell[b] = (long long)cell;
+    ptr[b] = (int)(blk_base >> 32) + wave_eoff[w] + upto - n;
     atomicExch(&cellmap[cell], b);
   }
 }
@@ -249,40 +269,60 @@ struct BandMacroArgs {
   double *band_u;
 };
 
-// every entry: its band cell and a slot among the cell's entries (the slots
-// are in arrival order; k_ibm_rank restores entry order).  A cell without a
-// band number would be an inconsistent build: reported in ctl[kErr] (code 4),
-// the entry skipped.  Thread b < nband also forms band cell b's velocity
-// from the stored state (k_band_macro's value).
-__global__ __launch_bounds__(256) void k_ibm_count(int E, const unsigned *__restrict__ keys,
-                                                   const int *__restrict__ cellmap, int *__restrict__ bidx,
-                                                   int *__restrict__ count, int *__restrict__ slot,
-                                                   int *__restrict__ ctl, BandMacroArgs ma) {
+// every entry: its band cell, and its place in the cell's range in arrival
+// order (k_ibm_rank restores entry order).  A cell without a band number would
+// be an inconsistent build: reported in ctl[kErr] (code 4), the entry skipped.
+// Thread b < nband also forms band cell b's velocity from the stored state
+// (k_band_macro's value).  The last workgroup reduces the claim workgroups'
+// parts of the band's bounding box (nbox of them) into ctl[kBoxLo..kBoxHi+2]
+// and closes the entry list.
+__global__ __launch_bounds__(256) void k_ibm_fill(int E, const unsigned *__restrict__ keys,
+                                                  const int *__restrict__ cellmap,
+                                                  const int *__restrict__ slot, int *__restrict__ ptr,
+                                                  int *__restrict__ bidx, int *__restrict__ tmp,
+                                                  int *__restrict__ ctl, const int *__restrict__ blkbox, int nbox,
+                                                  BandMacroArgs ma) {
+  if (blockIdx.x == gridDim.x - 1) {
+    __shared__ int wbox[4][6];
+    const int lane = threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+    int r[6] = {0x7fffffff, 0x7fffffff, 0x7fffffff, -1, -1, -1};
+    for (int q = threadIdx.x; q < nbox; q += blockDim.x)
+#pragma unroll
+      for (int k = 0; k < 6; ++k) r[k] = k < 3 ? min(r[k], blkbox[6 * q + k]) : max(r[k], blkbox[6 * q + k]);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      int v = r[k];
+      for (int off = 32; off > 0; off >>= 1) {
+        const int o = __shfl_xor(v, off, 64);
+        v = k < 3 ? min(v, o) : max(v, o);
+      }
+      if (lane == 0) wbox[w][k] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < 6) {
+      const int k = threadIdx.x;
+      int v = wbox[0][k];
+      for (int q = 1; q < 4; ++q) v = k < 3 ? min(v, wbox[q][k]) : max(v, wbox[q][k]);
+      ctl[kBoxLo + k] = v;
+    }
+    if (threadIdx.x == 0) ptr[ctl[kNew]] = ctl[kNewEntries];
+    return;
+  }
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= E) return;
+  const int b = cellmap_load(&cellmap[keys[e]]);
+  const int sl = slot[e];
   if (e < ctl[kNew]) {
     if (ma.f) band_macro_cell(ma.f, ma.N, ma.cell[e], e, ma.cap, ma.hv0, ma.hv1, ma.hv2, ma.band_u);
     else band_macro32_cell(ma.g, ma.N, ma.cell[e], e, ma.cap, ma.hv0, ma.hv1, ma.hv2, ma.band_u);
   }
-  const int b = cellmap_load(&cellmap[keys[e]]);
   if (b < 0 || b >= E) {
     atomicMin(&ctl[kErr], 4);
     bidx[e] = 0;
-    slot[e] = 0;
     return;
   }
   bidx[e] = b;
-  slot[e] = atomicAdd(&count[b], 1);
-}
-
-// entries into their cells' CSR ranges in slot order (band_ptr: inclusive
-// scan of the counts, shifted by one)
-__global__ __launch_bounds__(256) void k_ibm_fill(int E, const int *__restrict__ bidx,
-                                                  const int *__restrict__ slot, const int *__restrict__ band_ptr,
-                                                  int *__restrict__ tmp) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= E) return;
-  tmp[band_ptr[bidx[e]] + slot[e]] = e;
+  tmp[ptr[b] + sl] = e;
 }
 
 // every entry at its rank in its cell's range (the number of the cell's
@@ -312,7 +352,8 @@ __global__ __launch_bounds__(256) void k_ibm_rank(int E, int *__restrict__ ctl, 
     for (int j = 0; j < 16; ++j) r += v[j] < e ? 1 : 0;
   }
   // the entry's three stencil weights and its marker, in the cells' order
-  went[p0 + r] = make_float4(wx, wy, wz, __int_as_float(m));
+  // (an entry without a cell of its own, an error already reported, may not fit)
+  if (r < n) went[p0 + r] = make_float4(wx, wy, wz, __int_as_float(m));
   if (ecell) ecell[e] = make_int4(b, p0, n, r);
 }
 
@@ -875,93 +916,6 @@ __global__ __launch_bounds__(kRoundsThreads, 2) void k_rounds(RoundsArgs a) {
     a.band_u[ec.x] = u1;
     a.band_u[cap + ec.x] = u2;
     a.band_u[2LL * cap + ec.x] = u3;
-  }
-}
-
-// Inclusive scan of the per-cell entry counts of the band's cells (ctl[kNew],
-// final after k_ibm_claim) into the CSR pointers ptr[1..] (ptr[0] = 0), one
-// 1024-thread workgroup: each thread reads a run of kScanRun counts into
-// registers at once (the reads are the scan's latency), the run totals are
-// scanned within each wave by lane shuffles and across the sixteen waves by
-// one wave, then the runs are written with their offsets; bands above 16384
-// cells take further passes.  Integer sums: the result does not depend on the
-// order.  The workgroup also reduces the claim workgroups' parts of the
-// band's bounding box (nbox of them) into ctl[kBoxLo..kBoxHi+2].
-constexpr int kScanRun = 16;  // (a multiple of 4: the runs are read as int4)
-__global__ __launch_bounds__(1024) void k_band_scan(int *__restrict__ ctl, const int *__restrict__ count,
-                                                     int *__restrict__ ptr, const int *__restrict__ blkbox,
-                                                     int nbox) {
-  __shared__ int wtot[16];
-  __shared__ int wbox[16][6];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  {
-    int r[6] = {0x7fffffff, 0x7fffffff, 0x7fffffff, -1, -1, -1};
-    for (int q = t; q < nbox; q += blockDim.x)
-#pragma unroll
-      for (int k = 0; k < 6; ++k) r[k] = k < 3 ? min(r[k], blkbox[6 * q + k]) : max(r[k], blkbox[6 * q + k]);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      int v = r[k];
-      for (int off = 32; off > 0; off >>= 1) {
-        const int o = __shfl_xor(v, off, 64);
-        v = k < 3 ? min(v, o) : max(v, o);
-      }
-      if (lane == 0) wbox[w][k] = v;
-    }
-  }
-  // the cells claimed in this call (k_ibm_rank copies this count to kNband only later)
-  const int n = ctl[kNew];
-  int carry = 0;
-  for (int base = 0; base < n; base += 1024 * kScanRun) {
-    const int lo = base + t * kScanRun;
-    int c[kScanRun];
-    if (lo < n) {
-      // the run in 16-byte reads (count holds kScanRun spare words past the band)
-      const int4 *q = reinterpret_cast<const int4 *>(count + lo);
-#pragma unroll
-      for (int j = 0; j < kScanRun / 4; ++j) {
-        const int4 v = q[j];
-        c[4 * j] = v.x; c[4 * j + 1] = v.y; c[4 * j + 2] = v.z; c[4 * j + 3] = v.w;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kScanRun; ++j)
-      if (!(lo + j < n)) c[j] = 0;
-    int s = 0;
-#pragma unroll
-    for (int j = 0; j < kScanRun; ++j) s += c[j];
-    int v = s;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int o = __shfl_up(v, off, 64);
-      if (lane >= off) v += o;
-    }
-    __syncthreads();  // (the previous pass is done with wtot)
-    if (lane == 63) wtot[w] = v;
-    __syncthreads();
-    if (w == 0) {
-      int x = lane < 16 ? wtot[lane] : 0;
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) {
-        const int o = __shfl_up(x, off, 64);
-        if (lane >= off) x += o;
-      }
-      if (lane < 16) wtot[lane] = x;
-    }
-    __syncthreads();
-    int run = carry + (v - s) + (w ? wtot[w - 1] : 0);
-#pragma unroll
-    for (int j = 0; j < kScanRun; ++j) {
-      run += c[j];
-      if (lo + j < n) ptr[lo + j + 1] = run;
-    }
-    carry += wtot[15];
-  }
-  __syncthreads();
-  if (t < 6) {
-    int r = wbox[0][t];
-    for (int q = 1; q < 16; ++q) r = t < 3 ? min(r, wbox[q][t]) : max(r, wbox[q][t]);
-    ctl[kBoxLo + t] = r;
   }
 }
 
