@@ -142,8 +142,7 @@ struct Ibm {
   int cap = 0;                               // 64*M, stride of the band arrays
   DevBuf<float> dEw;                         // 12*M
   DevBuf<float4> went;                       // per band entry (CSR order): rx, ry, rz, its marker
-  bool one_launch = false;                   // the forcing rounds in one launch (k_rounds), then:
-  DevBuf<int4> ecell;                        // per stencil entry: its cell, the cell's range, its rank in it
+  bool one_launch = false;                   // the build and the forcing rounds in one launch (k_couple), then:
   DevBuf<double> xch;                        // the markers' forces and residual terms, two copies
   DevBuf<unsigned> keys;                      // cell of each stencil entry
   DevBuf<int> tmp;                            // entries in arrival order per band cell
@@ -1497,14 +1496,19 @@ int fsil_time_steps(int h, int nsteps, double t0, double dt, double *total_ms) {
 
 // ---------------------------------------------------------------------------
 // immersed boundary
-// whether the forcing rounds run in one launch: its workgroups have to be
-// resident together
-static int ibm_rounds_rule(Ibm &I) {
+// the loop condition before the first round (Solidbody.f90:893-895)
+static int ibm_no_rounds(const Ibm &I) { return (I.ntol > 0 && 1e10 > I.dtol) ? 0 : 1; }
+// the coupling call's build and rounds in one launch: a plain call of few markers
+static bool ibm_one_launch(const Ibm &I) { return I.one_launch && !ibm_no_rounds(I) && !I.warm_mlp && !I.record; }
+// whether a body set can run that way: the launch's workgroups have to be
+// resident together, and the block is not so large that its collision hides
+// the call
+static int ibm_one_launch_rule(Ibm &I, long long cells) {
   int dev = 0, cus = 0;
   HIPCHK(hipGetDevice(&dev));
   HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  constexpr int per = kRoundsThreads / 64;
-  I.one_launch = I.M > 0 && I.M <= std::min(kRoundsMarkers, cus / kRoundsShare * per);
+  constexpr int per = kCoupleThreads / 64;
+  I.one_launch = I.M > 0 && cells <= kCoupleCells && I.M <= std::min(kCoupleMarkers, cus / kCoupleShare * per);
   if (const char *e = getenv("FSIL_ROUNDS"))
     if (atoi(e) == 0) I.one_launch = false;
   return 0;
@@ -1596,11 +1600,8 @@ int fsil_ibm_define_bodies(int h, int nbodies, const int *nmarkers, const int *n
   HIPCHK(I.dptr.ensure((size_t)I.cap + 1));
   HIPCHK(I.dcell.ensure(I.cap));
   HIPCHK(I.band_u.ensure(3 * (size_t)I.cap));
-  if (ibm_rounds_rule(I)) return 1;
-  if (I.one_launch) {
-    HIPCHK(I.ecell.ensure(I.cap));
-    HIPCHK(I.xch.ensure(8 * (size_t)I.M));
-  }
+  if (ibm_one_launch_rule(I, b->N)) return 1;
+  if (I.one_launch) HIPCHK(I.xch.ensure(8 * (size_t)I.M));
   HIPCHK(I.band_F.ensure(3 * (size_t)I.cap));
   HIPCHK(I.dstate.ensure(4));
   HIPCHK(I.tolpart.ensure(std::max(1, I.M)));  // per-marker |dV|_1
@@ -1671,7 +1672,7 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
     if (upload(I.elem_xc, elem_xc, 3 * (size_t)I.nelems, s)) return 1;
   }
   // UpdateElmtInterp_ (Solidbody.f90:760-867) and the band, on the device
-  const int done0 = (I.ntol > 0 && 1e10 > I.dtol) ? 0 : 1;
+  const int done0 = ibm_no_rounds(I);
   Mlp *net = nullptr;
   if (I.warm_mlp) {
     auto it = g_mlps.find(I.warm_mlp);
@@ -1682,11 +1683,13 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
   }
   // the guess needs the previous call's force (Eprev) and the skip within the loop's cap
   const int warm = (net && !done0 && I.have_prev && I.skip < I.ntol) ? 1 : 0;
-  // the plain loop in one launch where its workgroups fit (k_rounds)
-  const bool one_launch = I.one_launch && !done0 && !net && !I.record;
-  hipLaunchKernelGGL(k_ibm_reset, dim3(std::min(1024, (E + 255) / 256)), dim3(256), 0, s, I.ctl.p, I.dcell.p,
-                     I.cellmap.p, I.dstate.p, done0, warm, I.skip, I.Eforce.p, 3 * M);
-  HIPCHK(hipGetLastError());
+  // the build and the plain loop in one launch where its workgroups fit (k_couple)
+  const bool one_launch = ibm_one_launch(I);
+  if (!one_launch) {
+    hipLaunchKernelGGL(k_ibm_reset, dim3(std::min(1024, (E + 255) / 256)), dim3(256), 0, s, I.ctl.p, I.dcell.p,
+                       I.cellmap.p, I.dstate.p, done0, warm, I.skip, I.Eforce.p, 3 * M);
+    HIPCHK(hipGetLastError());
+  }
   StencilArgs sa{};
   sa.M = M;
   sa.Exyz = I.Exyz.p;
@@ -1703,23 +1706,23 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
   // ranges, entries placed in arrival order (I.tmp), then at their ranks
   sa.cellmap = I.cellmap.p;
   sa.slot = I.slot.p;
-  hipLaunchKernelGGL(k_ibm_stencil, dim3((M + 3) / 4), dim3(256), 0, s, sa);
-  const int nclaim = (E + kClaimThreads - 1) / kClaimThreads;
-  hipLaunchKernelGGL(k_ibm_claim, dim3(nclaim), dim3(kClaimThreads), 0, s, E, I.keys.p, I.slot.p, I.cellmap.p,
-                     I.dcell.p, I.dptr.p, b->yd, b->zd, I.blkbox.p, I.ctl.p);
-  HIPCHK(hipGetLastError());
   // calculate_interaction_force (Solidbody.f90:869-918): band velocity of the stored state with the placing
   const double hv0 = 0.5 * b->VF[0] * b->dh, hv1 = 0.5 * b->VF[1] * b->dh, hv2 = 0.5 * b->VF[2] * b->dh;
   BandMacroArgs ma{};
   ma.f = b->precision == 0 ? b->fA.p : nullptr;
   ma.g = b->precision == 0 ? nullptr : b->gA.p;
   ma.N = b->N; ma.cell = I.dcell.p; ma.cap = I.cap; ma.hv0 = hv0; ma.hv1 = hv1; ma.hv2 = hv2; ma.band_u = I.band_u.p;
-  hipLaunchKernelGGL(k_ibm_fill, dim3((E + 255) / 256 + 1), dim3(256), 0, s, E, I.keys.p, I.cellmap.p, I.slot.p,
-                     I.dptr.p, I.dbidx.p, I.tmp.p, I.ctl.p, I.blkbox.p, nclaim, ma);
-  HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_ibm_rank, dim3((E + 255) / 256), dim3(256), 0, s, E, I.ctl.p, I.dbidx.p, I.dptr.p, I.tmp.p,
-                     I.dEw.p, I.went.p, one_launch ? I.ecell.p : nullptr);
-  HIPCHK(hipGetLastError());
+  if (!one_launch) {
+    hipLaunchKernelGGL(k_ibm_stencil, dim3((M + 3) / 4), dim3(256), 0, s, sa);
+    const int nclaim = (E + kClaimThreads - 1) / kClaimThreads;
+    hipLaunchKernelGGL(k_ibm_claim, dim3(nclaim), dim3(kClaimThreads), 0, s, E, I.keys.p, I.slot.p, I.cellmap.p,
+                       I.dcell.p, I.dptr.p, b->yd, b->zd, I.blkbox.p, I.ctl.p);
+    hipLaunchKernelGGL(k_ibm_fill, dim3((E + 255) / 256 + 1), dim3(256), 0, s, E, I.keys.p, I.cellmap.p, I.slot.p,
+                       I.dptr.p, I.dbidx.p, I.tmp.p, I.ctl.p, I.blkbox.p, nclaim, ma);
+    hipLaunchKernelGGL(k_ibm_rank, dim3((E + 255) / 256), dim3(256), 0, s, E, I.ctl.p, I.dbidx.p, I.dptr.p, I.tmp.p,
+                       I.dEw.p, I.went.p);
+    HIPCHK(hipGetLastError());
+  }
   const double invh3p = 0.5 * dt * ((1.0 / b->dh) * (1.0 / b->dh) * (1.0 / b->dh)) / I.denIn;
   double dsum = 0.0;
   for (int body = 0; body < I.nbodies; ++body) dsum = dsum + (double)I.nmark[body];
@@ -1749,12 +1752,11 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
   mt.tl = I.tolpart.p; mt.dstate = I.dstate.p; mt.M = M; mt.ntol = I.ntol;
   mt.dsum = dsum; mt.Uref = I.Uref; mt.dtol = I.dtol; mt.skip = I.skip;
   if (one_launch) {
-    RoundsArgs ra{};
-    ra.M = M; ra.cap = I.cap; ra.ctl = I.ctl.p;
-    ra.Ew = I.dEw.p; ra.went = I.went.p; ra.ecell = I.ecell.p; ra.Evel = I.Evel.p; ra.Ea = I.Ea.p;
-    ra.invh3 = invh3p; ra.Eforce = I.Eforce.p; ra.band_u = I.band_u.p; ra.xch = I.xch.p; ra.mt = mt;
-    constexpr int per = kRoundsThreads / 64;
-    hipLaunchKernelGGL(k_rounds, dim3((M + per - 1) / per), dim3(kRoundsThreads), 0, s, ra);
+    CoupleArgs ca{};
+    ca.st = sa; ca.ma = ma; ca.cell = I.dcell.p; ca.ptr = I.dptr.p; ca.tmp = I.tmp.p; ca.went = I.went.p;
+    ca.Evel = I.Evel.p; ca.Ea = I.Ea.p; ca.invh3 = invh3p; ca.Eforce = I.Eforce.p; ca.xch = I.xch.p; ca.mt = mt;
+    constexpr int per = kCoupleThreads / 64;
+    hipLaunchKernelGGL(k_couple, dim3((M + per - 1) / per), dim3(kCoupleThreads), 0, s, ca);
     HIPCHK(hipGetLastError());
   }
   for (int it = 0; it < rounds && !one_launch; ++it) {

@@ -41,7 +41,7 @@ enum IbmCtl {
   kWarm = 10,      // learned warm start in use for this call
   kFallback = 11,  // 1: the warm start did not lower the residual, restart from zero; 2: restarted
   kDone0 = 12,     // the done word at the start of a loop (no iteration at all)
-  kArrived = 13,   // workgroups of k_rounds that reached its barriers so far
+  kArrived = 13,   // workgroups of k_couple that reached its barriers so far (0 between calls)
   kRan = 14,       // the last forcing round whose interpolation ran (-1: none)
   kGuess = 15,     // 1: the learned guess was applied in this call (kept on fallback)
   kSkip = 16,      // forcing rounds the applied guess stands for (0 without a guess)
@@ -100,7 +100,6 @@ __global__ __launch_bounds__(256) void k_ibm_reset(int *__restrict__ ctl, const 
     ctl[kNew] = 0;
     ctl[kNewEntries] = 0;
     ctl[kRan] = -1;
-    ctl[kArrived] = 0;
     ctl[kErr] = 0x7fffffff;
     ctl[kDone] = done0;
     // a learned guess stands for the first `skip` forcing rounds: the loop
@@ -135,14 +134,14 @@ struct StencilArgs {
 // indices, lanes 0..11 write the FP32 weights, lane s the cell of entry s, and
 // counts the entry into the cell map, where a cell of n entries so far holds
 // -1 - n (cells outside the band hold -1).
-__global__ __launch_bounds__(256) void k_ibm_stencil(StencilArgs a) {
-  const int s = threadIdx.x & 63;
-  const int m = blockIdx.x * 4 + ((int)threadIdx.x >> 6);
-  if (m >= a.M) return;
+// Returns the error code of the indices; lanes 0..11 get weight s of the
+// marker's 12 in wt.
+__device__ __forceinline__ int stencil_entry(const StencilArgs &a, int m, int s, unsigned &key, float &wt) {
   const int m0 = a.first_marker[m];
   const int sel[3] = {s >> 4, (s >> 2) & 3, s & 3};
   int cidx[3];
   int err = 0;
+  wt = 0.0f;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const int ii = (int)floor((a.Exyz[3LL * m0 + k] - a.org[k]) * a.invdh);
@@ -155,12 +154,22 @@ __global__ __launch_bounds__(256) void k_ibm_stencil(StencilArgs a) {
     const int e = trim4(idx, a.nd[k], ix, a.bc[2 * k], a.bc[2 * k + 1]);
     if (e && !err) err = e;
     cidx[k] = ix[sel[k]];
-    if ((s >> 2) == k) a.Ew[12LL * m + s] = (float)peskin4((double)((s & 3) - 1) - off);
+    if ((s >> 2) == k) wt = (float)peskin4((double)((s & 3) - 1) - off);
   }
+  key = ((unsigned)(cidx[0] - 1) * (unsigned)a.nd[1] + (unsigned)(cidx[1] - 1)) * (unsigned)a.nd[2] +
+        (unsigned)(cidx[2] - 1);
+  return err;
+}
+
+__global__ __launch_bounds__(256) void k_ibm_stencil(StencilArgs a) {
+  const int s = threadIdx.x & 63;
+  const int m = blockIdx.x * 4 + ((int)threadIdx.x >> 6);
+  if (m >= a.M) return;
+  unsigned key;
+  float wt;
+  const int err = stencil_entry(a, m, s, key, wt);
+  if (s < 12) a.Ew[12LL * m + s] = wt;
   if (s == 0 && err) atomicMin(&a.ctl[kErr], (m + 1) * 4 + err);
-  const unsigned key =
-      ((unsigned)(cidx[0] - 1) * (unsigned)a.nd[1] + (unsigned)(cidx[1] - 1)) * (unsigned)a.nd[2] +
-      (unsigned)(cidx[2] - 1);
   a.keys[64LL * m + s] = key;
   a.slot[64LL * m + s] = -1 - atomicSub(&a.cellmap[key], 1);
 }
@@ -328,12 +337,10 @@ __global__ __launch_bounds__(256) void k_ibm_fill(int E, const unsigned *__restr
 // every entry at its rank in its cell's range (the number of the cell's
 // entries below it, its range read sixteen entries at a time), so each cell
 // lists its entries in ascending e: went holds an entry's weights (rx, ry,
-// rz) and its marker, ecell (where k_rounds runs) an entry's cell, the cell's
-// range and the entry's rank in it; the band size is published
+// rz) and its marker; the band size is published
 __global__ __launch_bounds__(256) void k_ibm_rank(int E, int *__restrict__ ctl, const int *__restrict__ bidx,
                                                   const int *__restrict__ band_ptr, const int *__restrict__ tmp,
-                                                  const float *__restrict__ Ew, float4 *__restrict__ went,
-                                                  int4 *__restrict__ ecell) {
+                                                  const float *__restrict__ Ew, float4 *__restrict__ went) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e == 0) ctl[kNband] = ctl[kNew];
   if (e >= E) return;
@@ -354,7 +361,6 @@ __global__ __launch_bounds__(256) void k_ibm_rank(int E, int *__restrict__ ctl, 
   // the entry's three stencil weights and its marker, in the cells' order
   // (an entry without a cell of its own, an error already reported, may not fit)
   if (r < n) went[p0 + r] = make_float4(wx, wy, wz, __int_as_float(m));
-  if (ecell) ecell[e] = make_int4(b, p0, n, r);
 }
 
 // band macros: den/u of every band cell from the stored state, same
@@ -731,192 +737,405 @@ __global__ __launch_bounds__(256) void k_correct(int *__restrict__ ctl, int roun
                            pass_cap);
 }
 
-// All forcing rounds of a call in one launch, one wave per marker, for marker
-// counts whose workgroups are all resident at once (kRoundsShare).
-// Lane s of a wave holds the velocity of the band cell of the marker's entry
-// s and the cell's entries (weights and markers, the first kRoundEntries of
-// them in registers) for the whole loop, so a cell's correction is formed by
-// the wave of every marker whose stencil holds it and the only values that
-// cross workgroups are the markers' forces and residual terms: a round is one
-// exchange behind one barrier instead of two launches.  Every sum is formed in
-// the order of k_interp, band_cells_reduce and mdf_tl_sum, and every workgroup
-// makes the same stop test; workgroup 0 records it.
-// The exchange goes through device-scope atomics (the workgroups run on
-// several XCDs) in two copies taken in turn: a workgroup writes round r+2's
-// values only after all have passed barrier r+1, that is, have read round r's.
-// A wait is bounded by kRoundsWait; the call then fails.
-// Bound by the exchange: about 4.5 us per round (store, count, poll and load
-// across the XCDs 3, ordered sums 1) where two launches took 9.7.  Ten rounds:
-// 144 markers 97 -> 49 us; a whole coupling call of markers 0.9 x 0.7 cells
-// apart 198 -> 160 us (256 markers), 206 -> 181 (512); with 512 markers in a
-// few cells 1676 -> 863.
-struct RoundsArgs {
-  int M, cap;
-  int *ctl;
-  const float *Ew;
-  const float4 *went;
-  const int4 *ecell;
+// The band build and all forcing rounds of a call in one launch, one wave per
+// marker, for marker counts whose workgroups are all resident at once
+// (kCoupleShare); k_ibm_reset .. k_ibm_rank and the rounds' launches otherwise.
+// Build: the launches' steps with a barrier between them, an entry's values
+// staying in its lane's registers (marker m's wave, lane s: entry 64 m + s).
+// Rounds: the lane holds the velocity of its entry's band cell and the cell's
+// entries (weights and markers, the first kCoupleEntries of them in registers),
+// so a cell's correction is formed by the wave of every marker whose stencil
+// holds it and the only values that cross workgroups are the markers' forces and
+// residual terms: a round is one exchange behind one barrier.  Every sum is
+// formed in the order of k_interp, band_cells_reduce and mdf_tl_sum, and every
+// workgroup makes the same stop test; workgroup 0 records it.
+// What one workgroup writes and another reads in this launch goes through
+// device-scope atomics (the workgroups run on several XCDs) and is complete
+// before the writer is counted at the next barrier.  The rounds' exchange has
+// two copies taken in turn: a workgroup writes round r+2's values only after
+// all have passed barrier r+1, that is, have read round r's.
+// A wait is bounded by kCoupleWait; the call then fails.
+// Bound by the barriers and one wave's FP64 rate: 4.2 us per round (ordered sums
+// 1.0, barrier 1.6, values into LDS and the residual 0.8, correction 0.8) where
+// two launches took 9.7; the build 23 us (five barriers of 2, the stencil and
+// stored state 4, claim 2.4, placing 3) where its launches took 26 and five gaps.
+// Ten rounds of 144 markers with the build 68 us (launches: 123 and the gaps),
+// three rounds of 256 42 us.  A whole coupling call of markers 0.9 x 0.7 cells
+// apart, launches / one launch: 188 / 144 us (256 markers), 197 / 182 (512); with
+// 512 markers in a few cells 1637 / 795.
+struct CoupleArgs {
+  StencilArgs st;  // (keys, slot and Ew are not used)
+  BandMacroArgs ma;
+  long long *cell;  // the band's cells, first the previous call's
+  int *ptr, *tmp;
+  float4 *went;
   const double *Evel, *Ea;
   double invh3;
-  double *Eforce, *band_u;
+  double *Eforce;
   double *xch;  // [2][4][M]: h^-3 F dt / (2 rho) per axis, |dV|_1
   MdfTest mt;
 };
 
-constexpr int kRoundsThreads = 256;   // four markers per workgroup
-constexpr int kRoundEntries = 16;     // entries of a cell held in registers (a plane of markers a cell apart: all)
+constexpr int kCoupleThreads = 256;   // four markers per workgroup
+constexpr int kCoupleEntries = 16;    // entries of a cell held in registers (a plane of markers a cell apart: all)
 // Every workgroup of the launch waits for every other, so all have to be
-// resident together: at most half as many as the CUs, of which each holds two
-// (173 VGPRs), so the launches of a process's four hardware queues fit at once,
-// and other kernels beside them end by themselves.  The repeated corrections
-// grow with the markers per workgroup's share of a CU; at the line (512
-// markers on 256 CUs) the form is still the faster one by 6-12%.
-constexpr int kRoundsShare = 2;
-constexpr int kRoundsMarkers = 512;   // (the exchanged values are kept in LDS)
-constexpr long long kRoundsWait = 1000000000LL;  // ticks of the 100 MHz clock: 10 s
+// resident together: at most half as many as the CUs, of which each holds two,
+// so the launches of a process's four hardware queues fit at once, and other
+// kernels beside them end by themselves.  The repeated corrections grow with
+// the markers per workgroup's share of a CU; at the line (512 markers on 256
+// CUs) the form is still the faster one.
+constexpr int kCoupleShare = 2;
+// On large blocks the collision beside the call is the longer chain, and this
+// launch's workgroups keep CU slots from it.  us per step, launches / one
+// launch: 16x16 markers, four beam sub-steps, 5.9M cells FP64 553 / 493, FP32
+// 399 / 337; 14M cells 826 / 837 and 458 / 469; rigid, 3.6M cells 259 / 246,
+// 5.9M 386 / 393.
+constexpr long long kCoupleCells = 6LL << 20;
+constexpr int kCoupleMarkers = 512;   // (the exchanged values are kept in LDS)
+constexpr long long kCoupleWait = 1000000000LL;  // ticks of the 100 MHz clock: 10 s
 
-__device__ __forceinline__ double xload(const double *p) {
+template <class T>
+__device__ __forceinline__ T xload(const T *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void xstore(double *p, double v) {
+template <class T>
+__device__ __forceinline__ void xstore(T *p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(kRoundsThreads, 2) void k_rounds(RoundsArgs a) {
-  constexpr int NW = kRoundsThreads / 64, B = kRoundEntries;
-  __shared__ double t[NW][3][64];
-  __shared__ double fx[4][kRoundsMarkers];
+// Barrier `nth` (from 1) of a launch.  Arrival: this workgroup's stores have
+// reached memory, then it is counted; the wait ends when all workgroups are
+// (true), or late (false; an LDS word).
+__device__ __forceinline__ void couple_arrive(int *arrived) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool couple_wait(int *arrived, int nth, int *late) {
+  if (threadIdx.x == 0) {
+    const int want = (int)gridDim.x * nth;
+    const long long t0 = (long long)wall_clock64();
+    while (xload(arrived) < want) {
+      if ((long long)wall_clock64() - t0 > kCoupleWait) {
+        *late = 1;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+  }
+  __syncthreads();
+  return *late == 0;
+}
+__device__ __forceinline__ bool couple_barrier(int *arrived, int nth, int *late) {
+  couple_arrive(arrived);
+  return couple_wait(arrived, nth, late);
+}
+
+// ascending sort of sixteen values in registers (odd-even merges)
+__device__ __forceinline__ void sort16(int *v) {
+#pragma unroll
+  for (int lp = 0; lp < 4; ++lp)
+#pragma unroll
+    for (int lk = lp; lk >= 0; --lk)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int p = 1 << lp, k = 1 << lk, lo = k % p;  // (compare i and i + k where both lie in one 2p block)
+        if (i >= lo && (i - lo) % (2 * k) < k && i + k < 16 && i / (2 * p) == (i + k) / (2 * p)) {
+          const int x = min(v[i], v[i + k]), y = max(v[i], v[i + k]);
+          v[i] = x;
+          v[i + k] = y;
+        }
+      }
+}
+
+// lane `l`'s value (l a constant)
+__device__ __forceinline__ double lane_value(double v, int l) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l), hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
+  return __hiloint2double(hi, lo);
+}
+
+__global__ __launch_bounds__(kCoupleThreads, 2) void k_couple(CoupleArgs a) {
+  constexpr int NW = kCoupleThreads / 64, B = kCoupleEntries;
+  // the weights of all markers while the entry lists are made, then the
+  // interpolation terms and the exchanged values
+  __shared__ union {
+    float W[kCoupleMarkers][12];
+    struct {
+      double t[NW][3][64], fx[4][kCoupleMarkers + 1];  // (value M: zero)
+    } r;
+  } lds;
+  double(&t)[NW][3][64] = lds.r.t;
+  double(&fx)[4][kCoupleMarkers + 1] = lds.r.fx;
   __shared__ double part[4];
-  __shared__ int late;
+  __shared__ int wave_won[NW], wave_ent[NW], wbox[NW][6], late;
+  __shared__ unsigned long long blk_base;
   const int w = threadIdx.x >> 6, s = threadIdx.x & 63;
   const int m = blockIdx.x * NW + w;
-  const int M = a.M, cap = a.cap;
+  const int M = a.st.M, E = 64 * M;
   const bool on = m < M;
   const int me = on ? m : M - 1;  // (a spare wave follows the last marker and stores nothing)
+  const int e = 64 * me + s;
+  int *const ctl = a.st.ctl, *const cellmap = a.st.cellmap, *const arrived = &ctl[kArrived];
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
   if (threadIdx.x == 0) late = 0;
-  const int4 ec = a.ecell[64LL * me + s];
-  const float *W = a.Ew + 12LL * me;
-  const double rx = (double)W[s >> 4], ry = (double)W[4 + ((s >> 2) & 3)], rz = (double)W[8 + (s & 3)];
-  const MdfWords wd0 = mdf_words(a.ctl, a.mt.dstate);
-  // lane c < 3: component c of the marker
-  const int c = min(s, 2);
-  const double ev = a.Evel[3LL * me + c], am = a.Ea[me];
-  double ef = a.Eforce[3LL * me + c];
-  double u1 = a.band_u[ec.x], u2 = a.band_u[cap + ec.x], u3 = a.band_u[2LL * cap + ec.x];
-  const int n = ec.z;
-  const float4 *we = a.went + ec.y;
-  float4 q[B];
-#pragma unroll
-  for (int j = 0; j < B; ++j) {
-    q[j] = we[max(min(j, n - 1), 0)];
-    q[j].w = __int_as_float((int)min((unsigned)__float_as_int(q[j].w), (unsigned)(M - 1)));
+  // k_ibm_reset's work
+  {
+    const int nprev = ctl[kNband];
+    for (int i = blockIdx.x * kCoupleThreads + threadIdx.x; i < nprev; i += gridDim.x * kCoupleThreads)
+      xstore(&cellmap[a.cell[i]], -1);
+    const int k = threadIdx.x;
+    if (blockIdx.x == 0 && k < kCtlWords && k != kNband && k != kArrived)
+      xstore(&ctl[k], k < 3 || k == kErr ? 0x7fffffff : k < 6 || k == kRan ? -1 : 0);
+    if (first) a.mt.dstate[0] = 1e10;
   }
-  const int nmax = [&] {
-    int v = n;
-    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
-    return __builtin_amdgcn_readfirstlane(v);
-  }();
-  MdfWords wd = wd0;
-  for (int r = 0;; ++r) {
-    t[w][0][s] = ((u1 * rx) * ry) * rz;
-    t[w][1][s] = ((u2 * rx) * ry) * rz;
-    t[w][2][s] = ((u3 * rx) * ry) * rz;
-    wave_sync();
-    double *xo = a.xch + (long long)(r & 1) * 4 * M;
-    {
-      double v = 0.0;
-#pragma unroll 16
-      for (int k = 0; k < 64; ++k) v = v + t[w][c][k];
-      const double d = ev - v, F = d * am;
-      ef = ef + F;
-      const double d0 = __shfl(d, 0, 64), d1 = __shfl(d, 1, 64), d2 = __shfl(d, 2, 64);
-      if (on && s < 4) xstore(&xo[(long long)s * M + m], s < 3 ? F * a.invh3 : (fabs(d0) + fabs(d1)) + fabs(d2));
+  unsigned key;
+  float wt;
+  const int err = stencil_entry(a.st, me, s, key, wt);
+  if (on && s < 12) xstore(&a.st.Ew[12LL * m + s], wt);
+  const float fwx = __shfl(wt, s >> 4, 64), fwy = __shfl(wt, 4 + ((s >> 2) & 3), 64),
+              fwz = __shfl(wt, 8 + (s & 3), 64);
+  double u[3];
+  if (a.ma.f) band_macro_cell(a.ma.f, a.ma.N, key, 0, 1, a.ma.hv0, a.ma.hv1, a.ma.hv2, u);
+  else band_macro32_cell(a.ma.g, a.ma.N, key, 0, 1, a.ma.hv0, a.ma.hv1, a.ma.hv2, u);
+  const int c = min(s, 2);  // lane c < 3: component c of the marker
+  const double ev = a.Evel[3LL * me + c], am = a.Ea[me];
+  const double ref = a.mt.dstate[2];
+  if (!couple_barrier(arrived, 1, &late)) goto timeout;
+  {
+    // the entry counted into its cell
+    int slot = 1;
+    if (on) slot = -1 - atomicSub(&cellmap[key], 1);
+    if (on && s == 0 && err) atomicMin(&ctl[kErr], (m + 1) * 4 + err);
+    if (!couple_barrier(arrived, 2, &late)) goto timeout;
+    // k_ibm_claim's work
+    const bool won = on && slot == 0;
+    const int n0 = won ? -1 - xload(&cellmap[key]) : 0;
+    const unsigned long long mask = __ballot(won);
+    int upto = n0;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(upto, off, 64);
+      if (s >= off) upto += o;
     }
-    // every store of this workgroup has reached memory, then it is counted
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    {
+      const unsigned ny = a.st.nd[1], nz = a.st.nd[2], plane = ny * nz;
+      const unsigned x = key / plane, r = key - x * plane, y = r / nz;
+      const int v[3] = {(int)x, (int)y, (int)(r - y * nz)};
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        int lo = won ? v[k] : 0x7fffffff, hi = won ? v[k] : -1;
+        for (int off = 32; off > 0; off >>= 1) {
+          lo = min(lo, __shfl_xor(lo, off, 64));
+          hi = max(hi, __shfl_xor(hi, off, 64));
+        }
+        if (s == 0) {
+          wbox[w][k] = lo;
+          wbox[w][3 + k] = hi;
+        }
+      }
+    }
+    if (s == 63) {
+      wave_won[w] = __popcll(mask);
+      wave_ent[w] = upto;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-      __hip_atomic_fetch_add(&a.ctl[kArrived], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const int want = (int)gridDim.x * (r + 1);
-      const long long t0 = (long long)wall_clock64();
-      while (__hip_atomic_load(&a.ctl[kArrived], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want) {
-        if ((long long)wall_clock64() - t0 > kRoundsWait) {
-          late = 1;
-          break;
+      int nw = 0, ne = 0;
+      for (int k = 0; k < NW; ++k) {
+        nw += wave_won[k];
+        ne += wave_ent[k];
+      }
+      blk_base = nw ? atomicAdd(reinterpret_cast<unsigned long long *>(&ctl[kNew]),
+                                ((unsigned long long)ne << 32) | (unsigned long long)nw)
+                    : 0ULL;
+    }
+    if (threadIdx.x >= 64 && threadIdx.x < 70) {
+      const int k = threadIdx.x - 64;
+      int r = wbox[0][k];
+      for (int q = 1; q < NW; ++q) r = k < 3 ? min(r, wbox[q][k]) : max(r, wbox[q][k]);
+      if (k < 3) atomicMin(&ctl[kBoxLo + k], r);
+      else atomicMax(&ctl[kBoxLo + k], r);
+    }
+    __syncthreads();
+    if (won) {
+      int b = (int)(blk_base & 0xffffffffULL) + __popcll(mask & ((1ULL << s) - 1ULL));
+      int p = (int)(blk_base >> 32) + upto - n0;
+      for (int k = 0; k < w; ++k) {
+        b += wave_won[k];
+        p += wave_ent[k];
+      }
+      a.cell[b] = (long long)key;
+      xstore(&a.ptr[b], p);
+      atomicExch(&cellmap[key], b);
+    }
+    if (!couple_barrier(arrived, 3, &late)) goto timeout;
+    // k_ibm_fill's and k_ibm_rank's work
+    const int nband = xload(&ctl[kNew]);
+    int b = xload(&cellmap[key]);
+    const bool placed = b >= 0 && b < nband;
+    if (!placed) {
+      atomicMin(&ctl[kErr], 4);
+      b = 0;
+    }
+    const int p0 = xload(&a.ptr[b]), n = placed ? (b + 1 < nband ? xload(&a.ptr[b + 1]) : E) - p0 : 0;
+    if (first) {
+      ctl[kNband] = nband;
+      a.ptr[nband] = E;
+    }
+    if (on && placed) xstore(&a.tmp[p0 + slot], e);
+    for (int i = threadIdx.x; i < 12 * M; i += kCoupleThreads) lds.W[0][i] = xload(&a.st.Ew[i]);
+    if (!couple_barrier(arrived, 4, &late)) goto timeout;
+    int rank = 0, near[B];
+#pragma unroll
+    for (int j = 0; j < B; ++j) near[j] = j < n ? xload(&a.tmp[p0 + j]) : 0x7fffffff;
+#pragma unroll
+    for (int j = 0; j < B; ++j) rank += near[j] < e ? 1 : 0;
+    for (int j0 = B; j0 < n; j0 += 16) {
+      int v[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v[j] = xload(&a.tmp[p0 + min(j0 + j, n - 1)]);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) rank += j0 + j < n && v[j] < e ? 1 : 0;
+    }
+    if (on && placed && rank < n) {
+      const unsigned long long *q = reinterpret_cast<const unsigned long long *>(&a.went[p0 + rank]);
+      unsigned long long *o = const_cast<unsigned long long *>(q);
+      xstore(&o[0], ((unsigned long long)__float_as_uint(fwy) << 32) | __float_as_uint(fwx));
+      xstore(&o[1], ((unsigned long long)(unsigned)m << 32) | __float_as_uint(fwz));
+    }
+    // the cell's list: its entries in order, from the placed ones where all are
+    // in registers, else from the list itself once every workgroup has written
+    // its part (plain reads from then on)
+    const float4 *we = a.went + p0;
+    float4 q[B];
+    couple_arrive(arrived);
+    if (__syncthreads_or(n > B)) {
+      if (!couple_wait(arrived, 5, &late)) goto timeout;
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+#pragma unroll
+      for (int j = 0; j < B; ++j) {
+        q[j] = we[max(min(j, n - 1), 0)];
+        q[j].w = __int_as_float((int)min((unsigned)__float_as_int(q[j].w), (unsigned)(M - 1)));
+      }
+    } else {
+      sort16(near);
+#pragma unroll
+      for (int j = 0; j < B; ++j) {
+        const int x = j < n ? min(near[j], E - 1) : 0, k = x >> 6;
+        q[j] = make_float4(lds.W[k][(x >> 4) & 3], lds.W[k][4 + ((x >> 2) & 3)], lds.W[k][8 + (x & 3)],
+                           __int_as_float(k));
+      }
+    }
+    // (past the list's end: a zero value with zero weights, u - 0 = u)
+#pragma unroll
+    for (int j = 0; j < B; ++j)
+      if (j >= n) q[j] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(M));
+    __syncthreads();  // (the weights' LDS is the rounds' from here on)
+    if (threadIdx.x < 4) fx[threadIdx.x][M] = 0.0;
+
+    // the forcing rounds
+    const double rx = (double)fwx, ry = (double)fwy, rz = (double)fwz;
+    double ef = 0.0, u1 = u[0], u2 = u[1], u3 = u[2];
+    const int nmax = [&] {
+      int v = n;
+      for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
+      return __builtin_amdgcn_readfirstlane(v);
+    }();
+    for (int r = 0;; ++r) {
+      t[w][0][s] = ((u1 * rx) * ry) * rz;
+      t[w][1][s] = ((u2 * rx) * ry) * rz;
+      t[w][2][s] = ((u3 * rx) * ry) * rz;
+      wave_sync();
+      double *xo = a.xch + (long long)(r & 1) * 4 * M;
+      {
+        double v = 0.0, x[2][16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[0][k] = t[w][c][k];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {  // (sixteen terms read ahead of those added)
+          if (g < 3) {
+#pragma unroll
+            for (int k = 0; k < 16; ++k) x[(g + 1) & 1][k] = t[w][c][16 * (g + 1) + k];
+          }
+#pragma unroll
+          for (int k = 0; k < 16; ++k) v = v + x[g & 1][k];
         }
-        __builtin_amdgcn_s_sleep(1);
+        const double d = ev - v, F = d * am;
+        ef = ef + F;
+        const double d0 = lane_value(d, 0), d1 = lane_value(d, 1), d2 = lane_value(d, 2);
+        if (on && s < 4) xstore(&xo[(long long)s * M + m], s < 3 ? F * a.invh3 : (fabs(d0) + fabs(d1)) + fabs(d2));
+      }
+      if (!couple_barrier(arrived, 6 + r, &late)) goto timeout;
+      for (int i = threadIdx.x; i < M; i += kCoupleThreads) {
+        double v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = xload(&xo[(long long)k * M + i]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) fx[k][i] = v[k];
+      }
+      __syncthreads();
+      // the residual, in mdf_tl_sum's order (256 strided sums, wave trees, the four in order)
+      {
+        double p = 0.0;
+        for (int i = threadIdx.x; i < M; i += 256) p = p + fx[3][i];
+        p = wave_sum(p);
+        if (s == 0) part[w] = p;
+      }
+      // the correction of this lane's cell, its entries in order
+#pragma unroll
+      for (int h = 0; h < B; h += 8) {
+        if (h >= nmax) break;
+        double f[8][3];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          int k = __float_as_int(q[h + j].w);
+          asm volatile("" : "+v"(k));  // (no addresses kept across the rounds)
+          f[j][0] = fx[0][k]; f[j][1] = fx[1][k]; f[j][2] = fx[2][k];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const double qx = (double)q[h + j].x, qy = (double)q[h + j].y, qz = (double)q[h + j].z;
+          u1 = u1 - ((f[j][0] * qx) * qy) * qz;
+          u2 = u2 - ((f[j][1] * qx) * qy) * qz;
+          u3 = u3 - ((f[j][2] * qx) * qy) * qz;
+        }
+      }
+      for (int j0 = B; j0 < n; j0 += 8) {
+        float4 g[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) g[j] = we[min(j0 + j, n - 1)];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int k = (int)min((unsigned)__float_as_int(g[j].w), (unsigned)(M - 1));
+          const double qx = (double)g[j].x, qy = (double)g[j].y, qz = (double)g[j].z;
+          const double x1 = ((fx[0][k] * qx) * qy) * qz, x2 = ((fx[1][k] * qx) * qy) * qz,
+                       x3 = ((fx[2][k] * qx) * qy) * qz;
+          u1 = j0 + j < n ? u1 - x1 : u1;
+          u2 = j0 + j < n ? u2 - x2 : u2;
+          u3 = j0 + j < n ? u3 - x3 : u3;
+        }
+      }
+      __syncthreads();
+      double tol = 0.0;
+      for (int k = 0; k < 4; ++k) tol = tol + part[k];
+      if (first) mdf_decide(ctl, a.mt.dstate, tol, a.mt.dsum, a.mt.Uref, a.mt.ntol, a.mt.dtol, a.mt.skip,
+                            MdfWords{r, 0, 0, ref});
+      // (mdf_decide's condition without a learned guess, after r + 1 iterations)
+      if (!isfinite(tol) || !(r + 1 < a.mt.ntol && tol / (a.mt.dsum * a.mt.Uref) > a.mt.dtol)) {
+        if (first) ctl[kRan] = r;
+        break;
       }
     }
-    __syncthreads();
-    if (late) {
-      if (threadIdx.x == 0) atomicMin(&a.ctl[kErr], 2);
-      return;
+    if (on && s < 3) a.Eforce[3LL * m + s] = ef;
+    if (on && placed && rank == 0) {  // the cell's first entry
+      a.ma.band_u[b] = u1;
+      a.ma.band_u[a.ma.cap + b] = u2;
+      a.ma.band_u[2LL * a.ma.cap + b] = u3;
     }
-    for (int i = threadIdx.x; i < M; i += kRoundsThreads) {
-      double v[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) v[k] = xload(&xo[(long long)k * M + i]);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) fx[k][i] = v[k];
-    }
-    __syncthreads();
-    // the residual, in mdf_tl_sum's order (256 strided sums, wave trees, the four in order)
-    if (threadIdx.x < 256) {
-      double p = 0.0;
-      for (int i = threadIdx.x; i < M; i += 256) p = p + fx[3][i];
-      p = wave_sum(p);
-      if (s == 0) part[w] = p;
-    }
-    // the correction of this lane's cell, its entries in order
-#pragma unroll
-    for (int j = 0; j < B; ++j) {
-      if (j % 4 == 0 && j >= nmax) break;
-      // (the weights stay FP32 in their registers: widened copies and LDS
-      // addresses kept across the rounds would double them)
-      float4 g = q[j];
-      asm volatile("" : "+v"(g.x), "+v"(g.y), "+v"(g.z), "+v"(g.w));
-      const int k = __float_as_int(g.w);
-      const double qx = (double)g.x, qy = (double)g.y, qz = (double)g.z;
-      const double x1 = ((fx[0][k] * qx) * qy) * qz, x2 = ((fx[1][k] * qx) * qy) * qz,
-                   x3 = ((fx[2][k] * qx) * qy) * qz;
-      u1 = j < n ? u1 - x1 : u1;
-      u2 = j < n ? u2 - x2 : u2;
-      u3 = j < n ? u3 - x3 : u3;
-    }
-    for (int j0 = B; j0 < n; j0 += 8) {
-      float4 g[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) g[j] = we[min(j0 + j, n - 1)];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int k = (int)min((unsigned)__float_as_int(g[j].w), (unsigned)(M - 1));
-        const double qx = (double)g[j].x, qy = (double)g[j].y, qz = (double)g[j].z;
-        const double x1 = ((fx[0][k] * qx) * qy) * qz, x2 = ((fx[1][k] * qx) * qy) * qz,
-                     x3 = ((fx[2][k] * qx) * qy) * qz;
-        u1 = j0 + j < n ? u1 - x1 : u1;
-        u2 = j0 + j < n ? u2 - x2 : u2;
-        u3 = j0 + j < n ? u3 - x3 : u3;
-      }
-    }
-    __syncthreads();
-    double tol = 0.0;
-    for (int k = 0; k < 4; ++k) tol = tol + part[k];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      wd.iters = r;
-      mdf_decide(a.ctl, a.mt.dstate, tol, a.mt.dsum, a.mt.Uref, a.mt.ntol, a.mt.dtol, a.mt.skip, wd);
-    }
-    // (mdf_decide's condition without a learned guess, after r + 1 iterations)
-    if (!isfinite(tol) || !(r + 1 < a.mt.ntol && tol / (a.mt.dsum * a.mt.Uref) > a.mt.dtol)) {
-      if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl[kRan] = r;
-      break;
-    }
+    return;
   }
-  if (on && s < 3) a.Eforce[3LL * m + s] = ef;
-  if (on && ec.w == 0) {  // the cell's first entry
-    a.band_u[ec.x] = u1;
-    a.band_u[cap + ec.x] = u2;
-    a.band_u[2LL * cap + ec.x] = u3;
-  }
+timeout:
+  if (threadIdx.x == 0) atomicMin(&ctl[kErr], 2);
 }
 
 // The control words and the last residual of a coupling call, written into
@@ -944,7 +1163,7 @@ struct IbmReport {
 constexpr int kLoadChunk = 256;
 
 struct IbmFinishArgs {
-  const int *ctl;
+  int *ctl;
   const double *dstate;
   IbmReport *rep;
   int cap;
@@ -994,6 +1213,7 @@ __global__ __launch_bounds__(256) void k_ibm_finish(IbmFinishArgs a) {
   }
   const int blk = (int)blockIdx.x - a.dof_blocks;
   if (blk == 0 && threadIdx.x < kCtlWords) a.rep->ctl[threadIdx.x] = a.ctl[threadIdx.x];
+  if (blk == 0 && threadIdx.x == 0) a.ctl[kArrived] = 0;
   if (blk == 0 && threadIdx.x == 0) a.rep->dmax = a.dstate[0];
   band_cells_reduce<true>(blk, a.ctl[kNband], a.band_blocks, a.cap, a.ptr, a.went, a.Eforce, a.invh3, a.band_F,
                           a.VF1, a.VF2, a.VF3, a.pass_cap);
