@@ -513,22 +513,31 @@ int launch_faces(Block &b, bool after_collide) {
   return 0;
 }
 
+// The two copies of a block's state, and what of it the device's last-level cache holds.
+constexpr double kCachedState = 268.4e6;
+double state_bytes(const Block &b) { return 2.0 * Q * (double)b.N * (b.precision == 0 ? 8.0 : 4.0); }
+
 // Workgroup of the cell kernels.  Rows of up to kCellThreads cells: whole
 // z-rows (the z-moving values are then exchanged inside the workgroup), as
-// many as fit 256 threads, and more where that raises the part of the waves'
-// lanes in use by over 7% (133-cell rows: three, 399 of 448 lanes, 360 us for
-// 301x149x133 FP64 where one row fills 133 of 192 and takes 397; below that
-// larger workgroups gain nothing or, with the block in the caches, lose:
-// 128x96x80 LES 55.0 us with four rows, 52.1 with three).  Longer rows are
-// cut into the width of 256, 192 or 128 that leaves the fewest idle lanes.
+// many as fit 256 threads.  Where the state exceeds the caches, more rows if
+// that raises the part of the waves' lanes in use by over 7% (133-cell rows:
+// three, 399 of 448 lanes, 360 us for 301x149x133 FP64 where one row fills 133
+// of 192 and takes 397), or by over 25% for MRT, whose waves are bound by their
+// registers (180x140x133: three rows 117 us in FP32, one 134; 150x110x99 FP64:
+// three rows 134 us, two 121).  In the caches larger workgroups lose: FP32
+// 110x80x70 18.5 us with five rows, 16.1 with three, 150x110x99 40.5 and 37.2.
+// Longer rows are cut into the width of 256, 192 or 128 that leaves the fewest
+// idle lanes.
 dim3 cell_block(const Block &b) {
   if (b.zd <= kCellThreads) {
     int best = 0;
     double use = 0.0;
-    for (int ty = std::max(1, std::min(256 / b.zd, b.yd)); ty <= std::min(kCellThreads / b.zd, b.yd); ++ty) {
+    const double gain = b.model == 3 ? 1.25 : 1.07;
+    const int most = state_bytes(b) > kCachedState ? kCellThreads / b.zd : std::max(1, 256 / b.zd);
+    for (int ty = std::max(1, std::min(256 / b.zd, b.yd)); ty <= std::min(most, b.yd); ++ty) {
       const int n = b.zd * ty;
       const double u = (double)n / (double)((n + 63) / 64 * 64);
-      if (u > 1.07 * use) {
+      if (u > gain * use) {
         use = u;
         best = ty;
       }
@@ -552,6 +561,12 @@ int zrow_exchange(const Block &b, dim3 blk) {
   if ((int)blk.x != b.zd) return 0;
   // FP32 rows of whole waves: lane permutes, 80 bytes of LDS per wave (FSIL_ZROW=1 forces the LDS form)
   if (b.precision == 1 && b.zd % 64 == 0 && !(e && !strcmp(e, "1"))) return 2;
+  // The LDS form keeps stores from being split between rows' ends; for a block
+  // in the caches it brings nothing unless it lets the z faces ride along (us
+  // per step with / without: periodic FP32 34x30x31 4.18 / 3.83, 80x60x50 9.04 /
+  // 8.83, 150x110x99 37.2 / 36.7, above the caches FP64 128x96x80 49.2 / 51.4;
+  // open faces FP32 34x30x31 14.9 / 17.6, 128x96x80 28.6 / 34.9).
+  if (!(e && !strcmp(e, "1")) && state_bytes(b) <= kCachedState && b.bc[4] == BC_PERIODIC && b.bc[5] == BC_PERIODIC) return 0;
   return 1;
 }
 
