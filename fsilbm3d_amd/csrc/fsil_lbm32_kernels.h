@@ -3,7 +3,7 @@
 // Storage: g_q = f_q - w_q in FP32 (half the bytes of the FP64 form).  The
 // deviations are O(1e-2) where f is O(1e-1), so FP32 keeps ~3 more significant
 // bits of the physical signal than storing f itself would.  The density
-// deviation and momentum are accumulated with compensated (Kahan) sums; the
+// deviation and momentum are summed in FP64 over opposite-direction pairs; the
 // collision works on deviations:
 //   feq_q - w_q = w_q * (drho + rho*(3 u.e + 4.5 (u.e)^2 - 1.5 u.u))
 //   g'_q = g_q + Omega*((feq_q - w_q) - g_q) + (1 - Omega/2) * Flb_q
