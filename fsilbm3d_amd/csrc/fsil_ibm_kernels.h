@@ -45,6 +45,7 @@ enum IbmCtl {
   kRan = 14,       // the last forcing round whose interpolation ran (-1: none)
   kGuess = 15,     // 1: the learned guess was applied in this call (kept on fallback)
   kSkip = 16,      // forcing rounds the applied guess stands for (0 without a guess)
+  kListed = 17,    // workgroups of k_couple whose part of the entry lists is written (0 between calls)
   kNew = 18,       // band cells claimed so far in this call (becomes kNband)
   kNewEntries = 19,  // and their entries (one 64-bit counter with kNew)
   kCtlWords = 20
@@ -751,7 +752,12 @@ __global__ __launch_bounds__(256) void k_correct(int *__restrict__ ctl, int roun
 // workgroup makes the same stop test; workgroup 0 records it.
 // What one workgroup writes and another reads in this launch goes through
 // device-scope atomics (the workgroups run on several XCDs) and is complete
-// before the writer is counted at the next barrier.  The rounds' exchange has
+// before the writer is counted at the next barrier.  The barriers share one
+// running count, so every workgroup waits at each of them: one that went on
+// would be counted for the next barrier in place of a workgroup that has yet to
+// reach this one.  The entry lists, for which only workgroups with a cell of
+// more than kCoupleEntries entries wait, are counted in a word of their own.
+// The rounds' exchange has
 // two copies taken in turn: a workgroup writes round r+2's values only after
 // all have passed barrier r+1, that is, have read round r's.
 // A wait is bounded by kCoupleWait; the call then fails.
@@ -803,9 +809,10 @@ __device__ __forceinline__ void xstore(T *p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Barrier `nth` (from 1) of a launch.  Arrival: this workgroup's stores have
-// reached memory, then it is counted; the wait ends when all workgroups are
-// (true), or late (false; an LDS word).
+// Arrival: this workgroup's stores have reached memory, then it is counted.
+// The wait ends when all workgroups are counted for the nth time (from 1: true),
+// which holds only if none can be counted for nth + 1 before that, or late
+// (false; an LDS word).
 __device__ __forceinline__ void couple_arrive(int *arrived) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -884,7 +891,7 @@ __global__ __launch_bounds__(kCoupleThreads, 2) void k_couple(CoupleArgs a) {
     for (int i = blockIdx.x * kCoupleThreads + threadIdx.x; i < nprev; i += gridDim.x * kCoupleThreads)
       xstore(&cellmap[a.cell[i]], -1);
     const int k = threadIdx.x;
-    if (blockIdx.x == 0 && k < kCtlWords && k != kNband && k != kArrived)
+    if (blockIdx.x == 0 && k < kCtlWords && k != kNband && k != kArrived && k != kListed)
       xstore(&ctl[k], k < 3 || k == kErr ? 0x7fffffff : k < 6 || k == kRan ? -1 : 0);
     if (first) a.mt.dstate[0] = 1e10;
   }
@@ -1008,9 +1015,9 @@ __global__ __launch_bounds__(kCoupleThreads, 2) void k_couple(CoupleArgs a) {
     // its part (plain reads from then on)
     const float4 *we = a.went + p0;
     float4 q[B];
-    couple_arrive(arrived);
+    couple_arrive(&ctl[kListed]);
     if (__syncthreads_or(n > B)) {
-      if (!couple_wait(arrived, 5, &late)) goto timeout;
+      if (!couple_wait(&ctl[kListed], 1, &late)) goto timeout;
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 #pragma unroll
       for (int j = 0; j < B; ++j) {
@@ -1065,7 +1072,7 @@ __global__ __launch_bounds__(kCoupleThreads, 2) void k_couple(CoupleArgs a) {
         const double d0 = lane_value(d, 0), d1 = lane_value(d, 1), d2 = lane_value(d, 2);
         if (on && s < 4) xstore(&xo[(long long)s * M + m], s < 3 ? F * a.invh3 : (fabs(d0) + fabs(d1)) + fabs(d2));
       }
-      if (!couple_barrier(arrived, 6 + r, &late)) goto timeout;
+      if (!couple_barrier(arrived, 5 + r, &late)) goto timeout;
       for (int i = threadIdx.x; i < M; i += kCoupleThreads) {
         double v[4];
 #pragma unroll
@@ -1213,7 +1220,7 @@ __global__ __launch_bounds__(256) void k_ibm_finish(IbmFinishArgs a) {
   }
   const int blk = (int)blockIdx.x - a.dof_blocks;
   if (blk == 0 && threadIdx.x < kCtlWords) a.rep->ctl[threadIdx.x] = a.ctl[threadIdx.x];
-  if (blk == 0 && threadIdx.x == 0) a.ctl[kArrived] = 0;
+  if (blk == 0 && threadIdx.x == 0) a.ctl[kArrived] = a.ctl[kListed] = 0;
   if (blk == 0 && threadIdx.x == 0) a.rep->dmax = a.dstate[0];
   band_cells_reduce<true>(blk, a.ctl[kNband], a.band_blocks, a.cap, a.ptr, a.went, a.Eforce, a.invh3, a.band_F,
                           a.VF1, a.VF2, a.VF3, a.pass_cap);
