@@ -144,6 +144,7 @@ struct Ibm {
   DevBuf<float4> went;                       // per band entry (CSR order): rx, ry, rz, its marker
   bool one_launch = false;                   // the build and the forcing rounds in one launch (k_couple), then:
   DevBuf<double> xch;                        // the markers' forces and residual terms, two copies
+  int couple_give_up = 0;                    // the barrier at which it gives up (FSIL_COUPLE_LATE, for tests)
   DevBuf<unsigned> keys;                      // cell of each stencil entry
   DevBuf<int> tmp;                            // entries in arrival order per band cell
   DevBuf<int> blkbox;                         // per claim workgroup: its part of the band's box
@@ -1526,6 +1527,7 @@ static int ibm_one_launch_rule(Ibm &I, long long cells) {
   I.one_launch = I.M > 0 && cells <= kCoupleCells && I.M <= std::min(kCoupleMarkers, cus / kCoupleShare * per);
   if (const char *e = getenv("FSIL_ROUNDS"))
     if (atoi(e) == 0) I.one_launch = false;
+  if (const char *e = getenv("FSIL_COUPLE_LATE")) I.couple_give_up = atoi(e);
   return 0;
 }
 
@@ -1770,6 +1772,7 @@ int fsil_ibm_interaction_force(int h, double dt, const double *Exyz, const doubl
     CoupleArgs ca{};
     ca.st = sa; ca.ma = ma; ca.cell = I.dcell.p; ca.ptr = I.dptr.p; ca.tmp = I.tmp.p; ca.went = I.went.p;
     ca.Evel = I.Evel.p; ca.Ea = I.Ea.p; ca.invh3 = invh3p; ca.Eforce = I.Eforce.p; ca.xch = I.xch.p; ca.mt = mt;
+    ca.give_up = I.couple_give_up;
     constexpr int per = kCoupleThreads / 64;
     hipLaunchKernelGGL(k_couple, dim3((M + per - 1) / per), dim3(kCoupleThreads), 0, s, ca);
     HIPCHK(hipGetLastError());
@@ -1913,6 +1916,14 @@ int ibm_check_report(Block &b) {
   if (err != 0x7fffffff) {
     I.active = false;
     if (err == 3) return fail("Nan found in PenaltyForce");
+    if (band_build_failed(err)) {
+      // the next call starts from a clear cell map, and without the one launch
+      // if its workgroups did not all run
+      I.have_box = false;
+      if (err == 2) I.one_launch = false;
+      HIPCHK(hipMemsetAsync(I.cellmap.p, 0xff, (size_t)b.N * sizeof(int), b.stream));  // -1
+      HIPCHK(hipStreamSynchronize(b.stream));
+    }
     if (err == 2) return fail("forcing rounds: a workgroup did not start in time");
     if (err == 4) return fail("immersed-boundary band: a stencil cell without a band number");
     const int m = err / 4 - 1, why = err % 4;

@@ -35,7 +35,8 @@ enum IbmCtl {
   kBoxLo = 0,      // [0..2] lowest band cell coordinate per axis (the fluid kernels look
   kBoxHi = 3,      // [3..5] highest       up the cell map only inside this box)
   kNband = 6,      // number of band cells
-  kErr = 7,        // first failing marker (1-based) * 4 + reason, INT_MAX when none
+  kErr = 7,        // first failing marker (1-based) * 4 + reason, INT_MAX when none (2: a late
+                   // workgroup of k_couple, 3: not a number, 4: inconsistent band build)
   kDone = 8,       // multi-direct-forcing loop finished
   kIters = 9,      // iterations run
   kWarm = 10,      // learned warm start in use for this call
@@ -50,6 +51,11 @@ enum IbmCtl {
   kNewEntries = 19,  // and their entries (one 64-bit counter with kNew)
   kCtlWords = 20
 };
+
+// whether an error word tells of a band build that did not complete (a late
+// workgroup of k_couple, an inconsistent build): the cell map then holds more
+// than the band's cells
+__host__ __device__ constexpr bool band_build_failed(int err) { return err == 2 || err == 4; }
 
 static_assert(kErr == kBandErrWord, "the fused kernels read the coupling error word at kBandErrWord");
 
@@ -280,8 +286,9 @@ struct BandMacroArgs {
 };
 
 // every entry: its band cell, and its place in the cell's range in arrival
-// order (k_ibm_rank restores entry order).  A cell without a band number would
-// be an inconsistent build: reported in ctl[kErr] (code 4), the entry skipped.
+// order (k_ibm_rank restores entry order).  A cell without a band number or a
+// place outside the list would be an inconsistent build: reported in ctl[kErr]
+// (code 4), the entry skipped.
 // Thread b < nband also forms band cell b's velocity from the stored state
 // (k_band_macro's value).  The last workgroup reduces the claim workgroups'
 // parts of the band's bounding box (nbox of them) into ctl[kBoxLo..kBoxHi+2]
@@ -326,13 +333,14 @@ __global__ __launch_bounds__(256) void k_ibm_fill(int E, const unsigned *__restr
     if (ma.f) band_macro_cell(ma.f, ma.N, ma.cell[e], e, ma.cap, ma.hv0, ma.hv1, ma.hv2, ma.band_u);
     else band_macro32_cell(ma.g, ma.N, ma.cell[e], e, ma.cap, ma.hv0, ma.hv1, ma.hv2, ma.band_u);
   }
-  if (b < 0 || b >= E) {
+  const int at = b >= 0 && b < E && sl >= 0 ? ptr[b] + sl : -1;
+  if (at < 0 || at >= E) {
     atomicMin(&ctl[kErr], 4);
     bidx[e] = 0;
     return;
   }
   bidx[e] = b;
-  tmp[ptr[b] + sl] = e;
+  tmp[at] = e;
 }
 
 // every entry at its rank in its cell's range (the number of the cell's
@@ -760,7 +768,9 @@ __global__ __launch_bounds__(256) void k_correct(int *__restrict__ ctl, int roun
 // The rounds' exchange has
 // two copies taken in turn: a workgroup writes round r+2's values only after
 // all have passed barrier r+1, that is, have read round r's.
-// A wait is bounded by kCoupleWait; the call then fails.
+// A wait is bounded by kCoupleWait; the call then fails, k_ibm_finish leaves
+// an empty band and the host clears the cell map, whose counts and numbers no
+// longer match the band, and takes the launches from then on.
 // Bound by the barriers and one wave's FP64 rate: 4.2 us per round (ordered sums
 // 1.0, barrier 1.6, values into LDS and the residual 0.8, correction 0.8) where
 // two launches took 9.7; the build 23 us (five barriers of 2, the stencil and
@@ -780,6 +790,7 @@ struct CoupleArgs {
   double *Eforce;
   double *xch;  // [2][4][M]: h^-3 F dt / (2 rho) per axis, |dV|_1
   MdfTest mt;
+  int give_up;  // the barrier whose waits fail at once (0: none; for tests)
 };
 
 constexpr int kCoupleThreads = 256;   // four markers per workgroup
@@ -812,30 +823,34 @@ __device__ __forceinline__ void xstore(T *p, T v) {
 // Arrival: this workgroup's stores have reached memory, then it is counted.
 // The wait ends when all workgroups are counted for the nth time (from 1: true),
 // which holds only if none can be counted for nth + 1 before that, or late
-// (false; an LDS word).
+// (false).
+struct CoupleLate {  // (LDS)
+  int give_up, late;
+};
 __device__ __forceinline__ void couple_arrive(int *arrived) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0) __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ bool couple_wait(int *arrived, int nth, int *late) {
+__device__ __forceinline__ bool couple_wait(int *arrived, int nth, CoupleLate *c) {
   if (threadIdx.x == 0) {
     const int want = (int)gridDim.x * nth;
     const long long t0 = (long long)wall_clock64();
-    while (xload(arrived) < want) {
-      if ((long long)wall_clock64() - t0 > kCoupleWait) {
-        *late = 1;
+    const bool give_up = nth == c->give_up;
+    while (give_up || xload(arrived) < want) {
+      if (give_up || (long long)wall_clock64() - t0 > kCoupleWait) {
+        c->late = 1;
         break;
       }
       __builtin_amdgcn_s_sleep(1);
     }
   }
   __syncthreads();
-  return *late == 0;
+  return c->late == 0;
 }
-__device__ __forceinline__ bool couple_barrier(int *arrived, int nth, int *late) {
+__device__ __forceinline__ bool couple_barrier(int *arrived, int nth, CoupleLate *c) {
   couple_arrive(arrived);
-  return couple_wait(arrived, nth, late);
+  return couple_wait(arrived, nth, c);
 }
 
 // ascending sort of sixteen values in registers (odd-even merges)
@@ -874,7 +889,8 @@ __global__ __launch_bounds__(kCoupleThreads, 2) void k_couple(CoupleArgs a) {
   double(&t)[NW][3][64] = lds.r.t;
   double(&fx)[4][kCoupleMarkers + 1] = lds.r.fx;
   __shared__ double part[4];
-  __shared__ int wave_won[NW], wave_ent[NW], wbox[NW][6], late;
+  __shared__ int wave_won[NW], wave_ent[NW], wbox[NW][6];
+  __shared__ CoupleLate late;
   __shared__ unsigned long long blk_base;
   const int w = threadIdx.x >> 6, s = threadIdx.x & 63;
   const int m = blockIdx.x * NW + w;
@@ -884,7 +900,7 @@ __global__ __launch_bounds__(kCoupleThreads, 2) void k_couple(CoupleArgs a) {
   const int e = 64 * me + s;
   int *const ctl = a.st.ctl, *const cellmap = a.st.cellmap, *const arrived = &ctl[kArrived];
   const bool first = blockIdx.x == 0 && threadIdx.x == 0;
-  if (threadIdx.x == 0) late = 0;
+  if (threadIdx.x == 0) late = CoupleLate{a.give_up, 0};
   // k_ibm_reset's work
   {
     const int nprev = ctl[kNband];
@@ -979,12 +995,11 @@ __global__ __launch_bounds__(kCoupleThreads, 2) void k_couple(CoupleArgs a) {
     // k_ibm_fill's and k_ibm_rank's work
     const int nband = xload(&ctl[kNew]);
     int b = xload(&cellmap[key]);
-    const bool placed = b >= 0 && b < nband;
-    if (!placed) {
-      atomicMin(&ctl[kErr], 4);
-      b = 0;
-    }
+    bool placed = b >= 0 && b < nband;
+    if (!placed) b = 0;
     const int p0 = xload(&a.ptr[b]), n = placed ? (b + 1 < nband ? xload(&a.ptr[b + 1]) : E) - p0 : 0;
+    placed = placed && (!on || (slot >= 0 && slot < n));
+    if (!placed) atomicMin(&ctl[kErr], 4);
     if (first) {
       ctl[kNband] = nband;
       a.ptr[nband] = E;
@@ -1028,7 +1043,7 @@ __global__ __launch_bounds__(kCoupleThreads, 2) void k_couple(CoupleArgs a) {
       sort16(near);
 #pragma unroll
       for (int j = 0; j < B; ++j) {
-        const int x = j < n ? min(near[j], E - 1) : 0, k = x >> 6;
+        const int x = j < n ? (int)min((unsigned)near[j], (unsigned)(E - 1)) : 0, k = x >> 6;
         q[j] = make_float4(lds.W[k][(x >> 4) & 3], lds.W[k][4 + ((x >> 2) & 3)], lds.W[k][8 + (x & 3)],
                            __int_as_float(k));
       }
@@ -1222,6 +1237,11 @@ __global__ __launch_bounds__(256) void k_ibm_finish(IbmFinishArgs a) {
   if (blk == 0 && threadIdx.x < kCtlWords) a.rep->ctl[threadIdx.x] = a.ctl[threadIdx.x];
   if (blk == 0 && threadIdx.x == 0) a.ctl[kArrived] = a.ctl[kListed] = 0;
   if (blk == 0 && threadIdx.x == 0) a.rep->dmax = a.dstate[0];
+  if (band_build_failed(a.ctl[kErr])) {  // (uniform) the band is left empty
+    if (blk == 0 && threadIdx.x <= kNband)
+      a.ctl[threadIdx.x] = threadIdx.x < 3 ? 0x7fffffff : (threadIdx.x < 6 ? -1 : 0);
+    return;
+  }
   band_cells_reduce<true>(blk, a.ctl[kNband], a.band_blocks, a.cap, a.ptr, a.went, a.Eforce, a.invh3, a.band_F,
                           a.VF1, a.VF2, a.VF3, a.pass_cap);
 }
