@@ -2867,18 +2867,8 @@ int mlp_blocks(int n) {
   return (ntile + per - 1) / per;
 }
 
-// k_mlp_rows takes more dynamic LDS than the default limit
-template <bool GRAD>
-int mlp_rows_lds() {
-  static const hipError_t e = hipFuncSetAttribute((const void *)k_mlp_rows<GRAD>,
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpGradLds));
-  HIPCHK(e);
-  return 0;
-}
-
 // FP32 forward of n samples into M.Yp
 int mlp_forward32(Mlp &M, const float *X, int n) {
-  if (mlp_rows_lds<false>()) return 1;
   hipLaunchKernelGGL(k_mlp_rows<false>, dim3(mlp_blocks(n)), dim3(kGradThreads), sizeof(MlpGradLds), M.s, X, nullptr,
                      nullptr, n, M.th.p, M.Yp.p, nullptr, nullptr);
   HIPCHK(hipGetLastError());
@@ -2888,7 +2878,6 @@ int mlp_forward32(Mlp &M, const float *X, int n) {
 // forward and backward of rows idx[0..n) (null: 0..n): the workgroups'
 // gradient parts into M.gpart, their squared errors into M.part
 int mlp_fwd_bwd(Mlp &M, const float *X, const float *Y, const int *idx, int n) {
-  if (mlp_rows_lds<true>()) return 1;
   M.nblk = mlp_blocks(n);
   HIPCHK(M.gpart.ensure((size_t)M.nblk * kMlpParams));
   HIPCHK(M.part.ensure(M.nblk));
@@ -2919,6 +2908,9 @@ int fsil_mlp_create(int seed, int *handle) {
   auto mp = std::make_unique<Mlp>();
   Mlp &M = *mp;
   HIPCHK(hipStreamCreateWithFlags(&M.s, hipStreamNonBlocking));
+  // k_mlp_rows takes more dynamic LDS than the default limit, which is a device's own
+  for (const void *k : {(const void *)k_mlp_rows<false>, (const void *)k_mlp_rows<true>})
+    HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(MlpGradLds)));
   std::vector<float> th(kMlpParams, 0.0f);
   const int sizes[4][2] = {{kMlpH, kMlpIn}, {kMlpH, kMlpH}, {kMlpH, kMlpH}, {kMlpOut, kMlpH}};
   int k = 0;
