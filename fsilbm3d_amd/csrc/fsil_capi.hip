@@ -253,7 +253,7 @@ struct Block {
   double tau = 1, Omega = 1, Omega2 = 1;
   int precision = 0;  // 0 FP64 plain, 1 FP32 deviation storage
   int nt = 0;         // population streams nontemporal (see stream_policy)
-  int zrow = 0;       // FP32 row exchange of the z-moving values (zrow_exchange), fixed at creation
+  int zrow = 0;       // row exchange of the z-moving values (zrow_exchange), fixed at creation
   ZFaces zf{};             // z faces that the collide launches apply
   bool rim = false;        // the other faces take one launch (k_rim)
   DevBuf<double> fA, fB;
@@ -514,7 +514,9 @@ int launch_faces(Block &b, bool after_collide) {
   return 0;
 }
 
-// The two copies of a block's state, and what of it the device's last-level cache holds.
+// The two copies of a block's state, and the size of the device's last-level
+// cache: the row rules below, measured at 248 MB and less and at 299 MB and
+// more, turn there (the streams' own line is stream_policy's).
 constexpr double kCachedState = 268.4e6;
 double state_bytes(const Block &b) { return 2.0 * Q * (double)b.N * (b.precision == 0 ? 8.0 : 4.0); }
 
@@ -605,11 +607,13 @@ size_t zrow_lds_bytes(int zrow, dim3 blk, size_t value) {
 // where the caches merge the partial lines that a launch stores: rows that
 // are not whole 128-byte lines (300x150x133 FP64: 399 us plain, 449
 // nontemporal), rows without the exchange up to 8 GiB per copy (384x192x192
-// FP64: 853 against 906; nontemporal is 3-14% faster above), and blocks whose
-// two copies stay in the 256 MB last-level cache (128x96x80 FP64, 299 MB: 49
-// against 54).  The rest, whole lines of larger blocks, streams nontemporally
-// (384x192x192 FP64: 788 against 808; 512x256x256: 1853 against 1929;
-// 200x120x64, 467 MB: 85.5 against 89.7; FP32 alike).
+// FP64: 853 against 906; nontemporal is 3-14% faster above), and blocks of
+// which the last-level cache holds enough from one step to the next: the line
+// lies at 200 MB per copy, between two copies of 299 MB, a little more than that
+// cache (128x96x80 FP64: 49 against 54), and of 467 MB (200x120x64: 89.7 against
+// 85.5).  The rest, whole lines of larger blocks, streams nontemporally
+// (384x192x192 FP64: 788 against 808; 512x256x256: 1853 against 1929; FP32
+// alike).
 // FSIL_STREAM_HINT=nt|plain overrides the choice (at block creation) for
 // tests that run both.
 int stream_policy(const Block &b) {
@@ -620,15 +624,6 @@ int stream_policy(const Block &b) {
   const double copy_bytes = (double)Q * (double)b.N * (double)value;
   if (b.zrow && (size_t)b.zd * value % 128 == 0) return copy_bytes > 200.0e6 ? 1 : 0;
   return copy_bytes > 8.0 * 1024 * 1024 * 1024 ? 1 : 0;
-}
-
-// (Coupled launches once streamed nontemporally to spare the beam kernel's
-// element data in the caches; that data now stays in the beam kernel's LDS,
-// and the block's own policy is measured faster: FP64 flexible plate 1.187 ->
-// 1.152 ms per step.)
-int stream_hint_for(const Block &b, bool band) {
-  (void)band;
-  return b.nt;
 }
 
 template <int MODEL>
@@ -674,7 +669,7 @@ int collide_stream(Block &b, int region = kRegionAll, const int *hole = nullptr)
   a.Mf = b.Mf.p;
   const bool force = (b.VF[0] != 0.0 || b.VF[1] != 0.0 || b.VF[2] != 0.0);
   const bool band = region != kRegionBulk && b.ibm.active && b.ibm.M > 0;
-  a.nt = stream_hint_for(b, band || region != kRegionAll);
+  a.nt = b.nt;
   if (band) {
     a.ctl = b.ibm.ctl.p;
     a.cellmap = b.ibm.cellmap.p;
@@ -756,7 +751,7 @@ int collide_stream32(Block &b, int region = kRegionAll, const int *hole = nullpt
   }
   const bool force = (b.VF[0] != 0.0 || b.VF[1] != 0.0 || b.VF[2] != 0.0);
   const bool band = region != kRegionBulk && b.ibm.active && b.ibm.M > 0;
-  a.nt = stream_hint_for(b, band || region != kRegionAll);
+  a.nt = b.nt;
   if (band) {
     a.ctl = b.ibm.ctl.p;
     a.cellmap = b.ibm.cellmap.p;
@@ -1087,10 +1082,11 @@ int fsil_block_create(int id, const int *dims, const double *geom, const int *bc
     // slots while the bulk's workgroups fill every CU.  The bulk asks for
     // enough LDS that at most R of its workgroups share a CU
     // (FSIL_BULK_RESIDENCY=R, default 3; 0: no limit): fewer leave the bulk
-    // short of waves, more starve the coupling.  Measured, ms for the same run
-    // at R = 2 and 3: FP64 31.0 and 30.6, sixty steps in FP32-deviation form
-    // 38.0 and 35.0 (at 4 and 5, with the faces still launches of their own:
-    // 32.4 and 33.7, 39.2 and 40.0).
+    // short of waves, more starve the coupling.  Measured at R = 2, 3 and 4 on
+    // one device, ms: thirty FP64 steps of the flexible plate (192-cell rows) 30.8,
+    // 30.1 and 31.1, sixty FP32-deviation steps 37.7, 34.1 and 35.9, twenty-four
+    // of the school (1024x384x384 FP32, 384-cell rows) with its flow to the host
+    // 167.6, 166.0 and 168.3.
     int R = 3;
     if (const char *r = getenv("FSIL_BULK_RESIDENCY")) R = atoi(r);
     int dev = 0, per_cu = 0;

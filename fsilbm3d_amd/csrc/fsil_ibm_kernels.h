@@ -765,9 +765,9 @@ __global__ __launch_bounds__(256) void k_correct(int *__restrict__ ctl, int roun
 // would be counted for the next barrier in place of a workgroup that has yet to
 // reach this one.  The entry lists, for which only workgroups with a cell of
 // more than kCoupleEntries entries wait, are counted in a word of their own.
-// The rounds' exchange has
-// two copies taken in turn: a workgroup writes round r+2's values only after
-// all have passed barrier r+1, that is, have read round r's.
+// The rounds' exchange has two copies taken in turn: a workgroup writes round
+// r+2's values only after all have passed barrier r+1, that is, have read round
+// r's.
 // A wait is bounded by kCoupleWait; the call then fails, k_ibm_finish leaves
 // an empty band and the host clears the cell map, whose counts and numbers no
 // longer match the band, and takes the launches from then on.
@@ -804,9 +804,11 @@ constexpr int kCoupleEntries = 16;    // entries of a cell held in registers (a 
 constexpr int kCoupleShare = 2;
 // On large blocks the collision beside the call is the longer chain, and this
 // launch's workgroups keep CU slots from it.  us per step, launches / one
-// launch: 16x16 markers, four beam sub-steps, 5.9M cells FP64 553 / 493, FP32
-// 399 / 337; 14M cells 826 / 837 and 458 / 469; rigid, 3.6M cells 259 / 246,
-// 5.9M 386 / 393.
+// launch, 225 markers, ten rounds and four beam sub-steps: 3.5M cells FP64 464 /
+// 405, FP32 367 / 307; 5.9M 540 / 478 and 387 / 326; 9.7M 741 / 744 and 495 /
+// 496.  Rigid, three rounds: 3.5M 265 / 249 and 172 / 157; 5.9M 376 / 383 and
+// 245 / 244; 9.7M 641 / 639 and 383 / 384.  The line lies where a flexible body
+// still gains 11-16%; a rigid one has lost its gain there.
 constexpr long long kCoupleCells = 6LL << 20;
 constexpr int kCoupleMarkers = 512;   // (the exchanged values are kept in LDS)
 constexpr long long kCoupleWait = 1000000000LL;  // ticks of the 100 MHz clock: 10 s

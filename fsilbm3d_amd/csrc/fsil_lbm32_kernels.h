@@ -278,7 +278,7 @@ __device__ __forceinline__ void collide_push32_cell(const Collide32Args &a, int 
 // workgroup's rows; rows past the block's last one take part idle).
 template <int MODEL, bool FORCE, bool BAND, bool NT>
 __global__ __launch_bounds__(kCellThreads) void k_collide_push32(Collide32Args a) {
-  // LDS of the exchange, sized at launch (zrow32_lds_bytes)
+  // LDS of the exchange, sized at launch (zrow_lds_bytes)
   extern __shared__ float zx[];
   if (a.region == kRegionHull) {
     for_hull_cells(a.ctl, a.hole, a.xd, a.yd, a.zd, [&](int x, int y, int z) {
