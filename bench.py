@@ -523,7 +523,7 @@ def main():
                     "roofline": {"bound": "hbm", "achieved": r64["achieved_gbs"], "peak": HBM_PEAK_GBS,
                                  "unit": "GB/s", "frac": r64["achieved_gbs"] / HBM_PEAK_GBS,
                                  "traffic": traffic_from_profiles(),
-                                 "kernel": "k_collide_push<1,false,false,false,false>", "kernel_ms": r64["kernel_ms"],
+                                 "kernel": "k_collide_push<1,false,false,false,true>", "kernel_ms": r64["kernel_ms"],
                                  "bytes_per_cell": B_CELL[0]}},
     }
     out["school"] = school

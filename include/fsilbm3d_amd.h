@@ -164,7 +164,10 @@ int fsil_ibm_set_params(int handle, int ntolLBM, double dtolLBM, double Uref, do
  * With Eforce, lodFlow, iters and dmax all NULL the call only queues its work
  * on the block's stream and returns (the fluid update and beam sub-steps that
  * follow are ordered after it on the device); its errors are then reported
- * by the next coupling call or fsil_ibm_forces. */
+ * by the next coupling call or fsil_ibm_forces.
+ * Up to 512 markers on blocks of up to 6*2^20 cells are one launch whose
+ * workgroups wait for each other, at most 10 s: past that the call fails, its
+ * band is empty, and the block's later calls take a launch per stage. */
 int fsil_ibm_interaction_force(int handle, double dt, const double *Exyz, const double *Evel,
                                const double *Ea, const double *elem_xc, double *Eforce,
                                double *lodFlow, int *iters, double *dmax);
